@@ -581,15 +581,15 @@ int ensure_c0(vsm_ctx *c, int maxs, int tw)
     return VSM_OK;
 }
 
-int record_halfstep(vsm_ctx *c, int maxs, int tw, const ViewDesc *dviews, const Tile *dtiles, int ntiles,
-                    const PMConst &pc, bool timed)
+int record_halfstep(vsm_ctx *c, int maxs, int tw, ViewDesc *dviews, int nviews, const Tile *dtiles,
+                    int ntiles, const PMConst &pc, bool timed)
 {
     {
         const int rc = ensure_c0(c, maxs, tw);
         if (rc) return rc;
     }
     if (timed) HIPCHK(c, hipEventRecord(c->ev0, c->stream));
-    HIPCHK(c, launch_halfstep(maxs, tw, dviews, dtiles, ntiles, pc, c->d_counters, c->d_work,
+    HIPCHK(c, launch_halfstep(maxs, tw, dviews, nviews, dtiles, ntiles, pc, c->d_counters, c->d_work,
                               grid_for(c, maxs, tw), c->d_c0, c->stream));
     if (timed) {
         HIPCHK(c, hipEventRecord(c->ev1, c->stream));
@@ -773,16 +773,15 @@ int batch_step(vsm_ctx *c, Batch &b, int k)
         for (auto &g : b.graphs)
             if (g.first == m) exec = g.second;
         if (!exec) {
-            // [zero the tile cursors, half-step, advance the device step
-            // counters] x m, captured once per length and replayed
+            // m half-steps (each leaves the tile cursors zero and advances the
+            // device step counters), captured once per length and replayed
             hipGraph_t graph = nullptr;
             HIPCHK(c, hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal));
             hipError_t ce = hipSuccess;
             for (int s = 0; s < m && ce == hipSuccess; ++s) {
-                ce = launch_halfstep(b.maxs, b.params.tile_width, b.dviews, b.dtiles, b.ntiles, pc,
-                                     c->d_counters, c->d_work, grid_for(c, b.maxs, b.params.tile_width),
-                                     c->d_c0, c->stream);
-                if (ce == hipSuccess) ce = launch_advance(b.dviews, (int)b.views.size(), c->stream);
+                ce = launch_halfstep(b.maxs, b.params.tile_width, b.dviews, (int)b.views.size(), b.dtiles,
+                                     b.ntiles, pc, c->d_counters, c->d_work,
+                                     grid_for(c, b.maxs, b.params.tile_width), c->d_c0, c->stream);
             }
             const hipError_t ee = hipStreamEndCapture(c->stream, &graph);
             if (ce != hipSuccess || ee != hipSuccess) {
@@ -808,10 +807,9 @@ int batch_step(vsm_ctx *c, Batch &b, int k)
         c->halfstep_launches += m;
     } else {
         for (int s = 0; s < m; ++s) {
-            const int rc = record_halfstep(c, b.maxs, b.params.tile_width, b.dviews, b.dtiles, b.ntiles, pc,
-                                           c->timing);
+            const int rc = record_halfstep(c, b.maxs, b.params.tile_width, b.dviews, (int)b.views.size(),
+                                           b.dtiles, b.ntiles, pc, c->timing);
             if (rc) return rc;
-            HIPCHK(c, launch_advance(b.dviews, (int)b.views.size(), c->stream));
         }
     }
     b.steps_done += m;
@@ -923,11 +921,12 @@ int vsm_create(int device, uint64_t hbm_budget_bytes, vsm_ctx **out)
         delete c;
         return VSM_EDEVICE;
     }
-    if (dalloc(c, &c->d_counters, 1) != VSM_OK || dalloc(c, &c->d_work, 8) != VSM_OK) {
+    if (dalloc(c, &c->d_counters, 1) != VSM_OK || dalloc(c, &c->d_work, kXcd + 1) != VSM_OK) {
         delete c;
         return VSM_ENOMEM;
     }
     (void)launch_fill_u64(reinterpret_cast<unsigned long long *>(c->d_counters), 4, 0ull, c->stream);
+    (void)launch_fill_u32(c->d_work, kXcd + 1, 0u, c->stream);
     (void)hipStreamSynchronize(c->stream);
     *out = c;
     return VSM_OK;
@@ -1274,7 +1273,7 @@ static int debug_state(vsm_ctx *c, const vsm_view_req *req, int pass, int mode, 
         const int nt = (int)tiles.size();
         if (mode == 0) HIPCHK(c, launch_init(dv, dt, nt, pc, 1, tw, c->stream));
         else if (mode == 1)
-            HIPCHK(c, launch_halfstep(V.n_src, tw, dv, dt, nt, pc, c->d_counters, c->d_work,
+            HIPCHK(c, launch_halfstep(V.n_src, tw, dv, 1, dt, nt, pc, c->d_counters, c->d_work,
                                       grid_for(c, V.n_src, tw), c->d_c0, c->stream));
         else HIPCHK(c, launch_filter(V.n_src, dv, dt, nt, pc, dm, c->stream));
         HIPCHK(c, hipMemcpyAsync(h.data(), vs.hyp, hw * sizeof(float4), hipMemcpyDeviceToHost, c->stream));
@@ -1997,7 +1996,7 @@ int vsm_serve_step(vsm_ctx *c, int32_t *n_active, int32_t *n_queued)
         // The descriptors and tiles stay on the device while a request is
         // active: a step re-concatenates the tile lists only when the active
         // list (or the tile width) changed, and the device step counters
-        // advance after each half-step (k_advance), in step with host_step.
+        // advance at the end of each half-step, in step with host_step.
         int maxs = 1, nslots = 0;
         for (ServeReq *r : c->active) {
             maxs = std::max(maxs, r->vs.desc.n_src);
@@ -2027,10 +2026,9 @@ int vsm_serve_step(vsm_ctx *c, int32_t *n_active, int32_t *n_queued)
             c->serve_dirty = false;
         }
         const PMConst pc = make_const(c->params);
-        if ((rc = record_halfstep(c, maxs, c->params.tile_width, c->serve_views, c->serve_tiles,
+        if ((rc = record_halfstep(c, maxs, c->params.tile_width, c->serve_views, nslots, c->serve_tiles,
                                   c->serve_ntiles, pc, c->timing)))
             return rc;
-        HIPCHK(c, launch_advance(c->serve_views, nslots, c->stream));
         HIPCHK(c, hipStreamSynchronize(c->stream));
         // Every active request has advanced one half-step.  The finished ones
         // leave the active list before any fallible work on them, so a

@@ -17,6 +17,7 @@ constexpr int kMaxSamples = 16;
 constexpr int kLdsW = kTileW + 2 * kMaxRadius;
 constexpr int kLdsH = kTileH + 2 * kMaxRadius;
 constexpr float kMaxCost = 2.0f;
+constexpr int kXcd = 8;           // MI355X: 8 XCDs, workgroups dispatched round-robin across them
 
 // Launch-wide constants (kernel argument).
 struct PMConst {

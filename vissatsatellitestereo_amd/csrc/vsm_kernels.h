@@ -8,7 +8,9 @@ namespace vsm {
 // Half-step kernel for up to maxs sources on tiles of tw x (512 / tw)
 // pixels: 16 or 32 wide, and 64 for at most 16 sources.
 bool tile_width_supported(int tw, int maxs);
-hipError_t launch_halfstep(int maxs, int tw, const ViewDesc *views, const Tile *tiles, int ntiles,
+// work: kXcd + 1 zeroed words, left zero; the half-step counters of
+// views[0 .. nadv-1] advance when the half-step is done.
+hipError_t launch_halfstep(int maxs, int tw, ViewDesc *views, int nadv, const Tile *tiles, int ntiles,
                            const PMConst &c, Counters *counters, unsigned int *work, int grid,
                            float *c0_scratch, hipStream_t st);
 // Resident workgroups of the persistent half-step kernel on this device.
@@ -29,7 +31,6 @@ hipError_t launch_finalize(const ViewDesc *views, int view, int npix, float *dep
                            float *cost, float *depth_keep, hipStream_t st);
 hipError_t launch_load_hyp(const ViewDesc *views, int view, int npix, const float *depth,
                            const float *normal, float cos_max_normal, hipStream_t st);
-hipError_t launch_advance(ViewDesc *views, int nviews, hipStream_t st);
 hipError_t launch_pack_depth4(const float *depth, int W, int H, float4 *out, hipStream_t st);
 hipError_t launch_pack_pair(const uint8_t *gray, int W, int H, uint16_t *pair, hipStream_t st);
 hipError_t launch_fill_u64(unsigned long long *p, int n, unsigned long long v, hipStream_t st);

@@ -1107,19 +1107,24 @@ __device__ __forceinline__ void halfstep_tile(const ViewDesc &V, const Tile &t, 
     }
 }
 
-constexpr int kXcd = 8;   // MI355X: 8 XCDs, workgroups dispatched round-robin across them
-
 // Persistent red-black half-step over a tile list.  Workgroup b runs on XCD
 // b % 8 and takes tiles from that XCD's contiguous share of the list (the
 // views' source images stay in that XCD's L2), then steals from the other
-// XCDs' shares.  work[8] are per-XCD cursors zeroed before the launch.  The
-// order tiles are taken in never changes a result: tiles are independent
-// within a half-step.
+// XCDs' shares.  The order tiles are taken in never changes a result: tiles
+// are independent within a half-step.
+//
+// work[0 .. kXcd-1] are the per-XCD cursors, work[kXcd] counts the workgroups
+// that are done: all zero before the first launch, and left zero by the last
+// workgroup to finish, which also advances the half-step counters of the views
+// (adv[0 .. nadv-1]).  Nothing else runs between two half-steps: a fill and an
+// advance kernel of 5 us each used to (photo solve of two 256 x 256 views, 10
+// half-steps: 1802 -> 1753 us).
 template <int MAXS, int TW>
 __global__ __launch_bounds__(kThreads, 2) void k_halfstep(const ViewDesc *__restrict__ views,
                                                        const Tile *__restrict__ tiles, int ntiles,
                                                        PMConst c, Counters *counters,
-                                                       unsigned int *work, float *c0g)
+                                                       unsigned int *work, float *c0g, ViewDesc *adv,
+                                                       int nadv)
 {
     __shared__ float s_ref[TileShape<TW>::LH * TileShape<TW>::LW];
     __shared__ SrcLds s_src[MAXS];
@@ -1163,6 +1168,15 @@ __global__ __launch_bounds__(kThreads, 2) void k_halfstep(const ViewDesc *__rest
             atomicAdd(&counters->ncc_evals, (unsigned long long)s_evals[0]);
             atomicAdd(&counters->geo_evals, (unsigned long long)s_evals[1]);
         }
+    }
+    // Every workgroup has read the cursors and the step counters for the last
+    // time when it adds itself here, so the last one alone owns them.
+    if (tid == 0) s_tile = atomicAdd(&work[kXcd], 1u) == gridDim.x - 1;
+    __syncthreads();
+    if (s_tile) {
+        if (tid <= kXcd) work[tid] = 0u;
+        for (int v = tid; v < nadv; v += kThreads)
+            if (adv[v].active && adv[v].step < adv[v].num_steps) adv[v].step += 1;
     }
 }
 
@@ -1497,13 +1511,6 @@ __global__ void k_load_hyp(const ViewDesc *__restrict__ views, int view, const f
     V.hyp[p] = make_float4(d, n0, n1, n2);
 }
 
-// Device-side schedule step: every active view advances one half-step.
-__global__ void k_advance(ViewDesc *views, int nviews)
-{
-    const int v = blockIdx.x * blockDim.x + threadIdx.x;
-    if (v < nviews && views[v].active && views[v].step < views[v].num_steps) views[v].step += 1;
-}
-
 // Pair texture: W + 1 texels of 2 bytes per row; texel (x, y) holds I(x', y)
 // and I(x', y1) with x' = min(x, W-1), y1 = min(y+1, H-1).  The word at texel
 // x < W is the bilinear quad of (x, y) with edge-clamped neighbours (bytes
@@ -1543,7 +1550,7 @@ __global__ void k_fill_u64(unsigned long long *p, int n, unsigned long long v)
 // The kernel instantiation for (sources, tile width); null for an
 // unsupported width.
 typedef void (*halfstep_fn)(const ViewDesc *, const Tile *, int, PMConst, Counters *, unsigned int *,
-                            float *);
+                            float *, ViewDesc *, int);
 
 template <int MAXS>
 static halfstep_fn halfstep_for_width(int tw)
@@ -1569,7 +1576,7 @@ static halfstep_fn halfstep_kernel(int maxs, int tw)
 
 bool tile_width_supported(int tw, int maxs) { return tw == 16 || tw == 32 || (tw == 64 && maxs <= 16); }
 
-hipError_t launch_halfstep(int maxs, int tw, const ViewDesc *views, const Tile *tiles, int ntiles,
+hipError_t launch_halfstep(int maxs, int tw, ViewDesc *views, int nadv, const Tile *tiles, int ntiles,
                            const PMConst &c, Counters *counters, unsigned int *work, int grid,
                            float *c0_scratch, hipStream_t st)
 {
@@ -1578,10 +1585,8 @@ hipError_t launch_halfstep(int maxs, int tw, const ViewDesc *views, const Tile *
     if (!fn) return hipErrorInvalidValue;
     // more than 16 sources: c0_scratch holds grid x 32 x kThreads floats
     if (maxs > 16 && !c0_scratch) return hipErrorInvalidValue;
-    hipError_t e = launch_fill_u32(work, kXcd, 0u, st);
-    if (e != hipSuccess) return e;
     grid = max(kXcd, min(grid, ((ntiles + kXcd - 1) / kXcd) * kXcd));
-    fn<<<grid, kThreads, 0, st>>>(views, tiles, ntiles, c, counters, work, c0_scratch);
+    fn<<<grid, kThreads, 0, st>>>(views, tiles, ntiles, c, counters, work, c0_scratch, views, nadv);
     return hipGetLastError();
 }
 
@@ -1652,12 +1657,6 @@ hipError_t launch_load_hyp(const ViewDesc *views, int view, int npix, const floa
                            const float *normal, float cos_max_normal, hipStream_t st)
 {
     k_load_hyp<<<(npix + 255) / 256, 256, 0, st>>>(views, view, depth, normal, cos_max_normal);
-    return hipGetLastError();
-}
-
-hipError_t launch_advance(ViewDesc *views, int nviews, hipStream_t st)
-{
-    k_advance<<<(nviews + 63) / 64, 64, 0, st>>>(views, nviews);
     return hipGetLastError();
 }
 
