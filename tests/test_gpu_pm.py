@@ -189,6 +189,29 @@ def test_lockstep_geometric_18_sources(many):
         assert r["frac_cost_err"] <= 1e-3, r
 
 
+@pytest.mark.parametrize("name,n_src,pass_,extra", [
+    ("many", 1, 0, {}),                                   # no source after the first to leave out
+    ("many", 2, 0, dict(draw_group=1, tile_width=16)),
+    ("many", 17, 0, dict(draw_group=1)),                  # the kernel for more than 16 sources
+    ("ragged", 3, 0, dict(tile_width=64)),                # waves with pixels outside the image
+    ("ragged", 3, 1, {}),
+    ("ragged", 3, 1, dict(geom_consistency_regularizer=-0.05)),   # sums may fall: every source counts
+    ("many", 9, 1, dict(draw_group=1, geom_consistency_max_cost=0.5)),
+])
+def test_lockstep_candidates_leave_early(many, ragged, name, n_src, pass_, extra):
+    """Candidates whose partial cost has reached the best complete one leave a
+    pixel's list, and idle lanes take over planes of busy ones: winners and
+    costs stay the oracle's, which evaluates every candidate on every drawn
+    source.  Six half-steps, so the current planes are good ones."""
+    site = dict(many=many, ragged=ragged)[name]
+    srcs = [n for n in site["names"] if n != site["names"][0]]
+    rep, _ = _lockstep(site, _params(window_radius=5, window_step=2, **extra), 0, n_src, pass_, 6,
+                       src_depths_gpu=_src_depths(site, srcs) if pass_ else None)
+    for r in rep:
+        assert r["decided_mismatch"] <= 1e-3, r
+        assert r["frac_cost_err"] <= 1e-3, r
+
+
 def test_lds_staged_costs_equal_cached(tiny):
     """The measurement kernel that reads window taps from LDS-staged boxes of
     the sources returns the same costs as its cached-gather twin and as

@@ -65,6 +65,7 @@ struct SrcLds {
     const float4 *depth4;        // photometric depth of the source, 2x2 per texel
     float ptri, tri, g0, g1, g2;
     int inner;                   // every window of the tile lies inside the source (see below)
+    int linear;                  // no window of the tile needs a per-tap reciprocal (see below)
 };
 
 struct Proj {
@@ -80,6 +81,25 @@ __device__ __forceinline__ float slope_bound(const PMConst &c)
 {
     const float cm = c.cos_max_normal;
     return cm > 0.f ? 1.01f * sqrtf(fmaxf(1.f - cm * cm, 0.f)) / cm : 0.f;
+}
+
+// Ranges of depth beyond hyp_depth_lo and hyp_depth_hi within which `linear`
+// holds: planes that extrapolate this far are all but never met.
+constexpr float kLinearRange = 8.f;
+
+// 1 when no window of a tile, under any hypothesis with depth in [dlo, dhi] and
+// slopes |a|, |b| <= amax, needs the per-tap reciprocal: the homogeneous depth,
+// affine over the box of the tile's taps, is positive at its corners and
+// delta <= kDeltaMax / 2 there.  A pass then takes the same variant whichever
+// of a wave's planes it evaluates.
+__device__ int source_linear(const double (&A)[12], double hu, double hv, double r, double dlo, double dhi,
+                             double amax)
+{
+    const double d0 = dlo - 2.0 * amax * r, d1 = dhi + 2.0 * amax * r;
+    const double side = fabs(A[8]) * (hu + r) + fabs(A[9]) * (hv + r);
+    const double zmin = fmin(A[11] * d0, A[11] * d1) + A[10] - side;
+    if (!(zmin > 0.0)) return 0;
+    return r * (fabs(A[8]) + fabs(A[9]) + 2.0 * amax * fabs(A[11])) / zmin <= 0.5 * (double)kDeltaMax ? 1 : 0;
 }
 
 // 1 when every tap of every window of a tile (pixel box hu x hv around the
@@ -164,6 +184,8 @@ __device__ void setup_source(const ViewDesc &V, const PMConst &c, int s, int uc,
         const double dhi = hyp_depth_hi(V) + 1e-3 * (fabs(dr) + 1.0);
         o.inner = source_inner(A, hu, hv, (double)c.radius, dlo, dhi, (double)slope_bound(c),
                                (double)o.lox, (double)o.hix, (double)o.loy, (double)o.hiy);
+        const double more = (double)kLinearRange * dr;
+        o.linear = source_linear(A, hu, hv, (double)c.radius, dlo - more, dhi + more, (double)slope_bound(c));
     }
 }
 
@@ -464,16 +486,20 @@ __device__ __forceinline__ void window_pass_r5s2(const PMConst &c, const SrcView
         giv[k] = -iz0[k] * iz0[k] * P[k].hvz;
         ss[k] = 0.f; sss[k] = 0.f; srs[k] = 0.f;
     }
+    // Register sets used in turn, so D - 1 taps' gathers are in flight while
+    // one is accumulated: a narrow pass has fewer gathers per tap and less
+    // arithmetic to cover their latency.
+    constexpr int D = G >= 3 ? 2 : G == 2 ? 3 : 6;
     float rx[G], ry[G], rz[G];
     row_start<G, false>(P, iz0, giu, giv, (float)(-RAD), -RAD, rx, ry, rz);
-    uint32_t v[2][G];
-    float fx[2][G], fy[2][G], rr[2], ww[2];
+    uint32_t v[D][G];
+    float fx[D][G], fy[D][G], rr[D], ww[D];
     const float *ref_row = s_ref + lbase - RAD * R.ldsw - RAD;    // row -RAD, column -RAD
     const float *wt_row = R.wt;
-    // gathers and LDS reads of tap ii of the current row into set ii & 1,
-    // after the accumulation that last used that set (tok)
+    // gathers and LDS reads of tap ii of the issue row into set ii % D, after
+    // the accumulation that last used that set (tok)
     auto issue = [&](int ii, const float (&tok)[G]) {
-        const int b = ii & 1;
+        const int b = ii % D;
         float fi = (float)(ii * ST);
 #pragma unroll
         for (int k = 0; k < G; ++k) asm volatile("" : "+v"(fi) : "v"(tok[k]));
@@ -486,7 +512,7 @@ __device__ __forceinline__ void window_pass_r5s2(const PMConst &c, const SrcView
         __builtin_amdgcn_s_setprio(0);
     };
     auto consume = [&](int ii) {
-        const int b = ii & 1;
+        const int b = ii % D;
         const float r = rr[b] - R.rc;
         const float w = ww[b];
         const float wr = w * r;
@@ -499,19 +525,22 @@ __device__ __forceinline__ void window_pass_r5s2(const PMConst &c, const SrcView
             srs[k] = fmaf(wr, sv, srs[k]);
         }
     };
-    issue(0, ss);
+#pragma unroll
+    for (int ii = 0; ii + 1 < D; ++ii) issue(ii, ss);
 #pragma unroll 1
     for (int jj = 0; jj < NT; ++jj) {
 #pragma unroll
         for (int ii = 0; ii < NT; ++ii) {
-            if (ii + 1 < NT) {
-                issue(ii + 1, ss);
+            const int nx = ii + D - 1;                // the tap to issue, in the next row from NT on
+            if (nx < NT) {
+                issue(nx, ss);
             } else if (jj + 1 < NT) {
-                // first tap of the next row into set 0 (free: tap 4 was accumulated)
-                row_start<G, false>(P, iz0, giu, giv, (float)(-RAD), -RAD + (jj + 1) * ST, rx, ry, rz);
-                ref_row += ST * R.ldsw;
-                wt_row += NT * kThreads;
-                issue(0, ss);
+                if (nx == NT) {
+                    row_start<G, false>(P, iz0, giu, giv, (float)(-RAD), -RAD + (jj + 1) * ST, rx, ry, rz);
+                    ref_row += ST * R.ldsw;
+                    wt_row += NT * kThreads;
+                }
+                issue(nx - NT, ss);
             }
             consume(ii);
         }
@@ -747,46 +776,72 @@ __device__ __forceinline__ void select_group(const PMConst &c, const SrcLds *s_s
     for (int k = 0; k < G; ++k) s_c0[(s0 + k) * kThreads + tid] = cg[k];
 }
 
-// Candidate hypotheses K0+1 .. K0+G against source Ss in one shared window
-// pass; acc[k] += cnt * cost (photometric, plus the geometric term in pass 1).
-template <int G, int K0>
-__device__ __forceinline__ void eval_hyp_group(const PMConst &c, const SrcLds &Ss, float cnt, int pass,
-                                               float du, float dv, const float (&hd)[kNHyp],
-                                               const float (&ak)[kNHyp - 1],
-                                               const float (&bk)[kNHyp - 1], const float *s_ref,
-                                               int lbase, const RefStats &R, float (&acc)[kNHyp - 1],
-                                               bool hyp_ok)
+// What a lane evaluates in one window pass: up to kGroupH planes (slopes a, b)
+// of one pixel, its own or another lane's.
+struct Unit {
+    float du, dv;
+    int lbase, n;                // n: planes of the unit, 0 for an idle lane
+    float d[kGroupH], a[kGroupH], b[kGroupH];
+    RefStats R;
+};
+
+// Costs of a unit's planes against source Ss in one shared window pass of G
+// slots: photometric, plus the geometric term in pass 1.  A lane with fewer
+// planes repeats its first one, whose gathers fall on lines the pass reads
+// anyway.
+template <int G>
+__device__ __forceinline__ void eval_unit(const PMConst &c, const SrcLds &Ss, int pass, const Unit &U,
+                                          const float *s_ref, float (&res)[kGroupH], bool hyp_ok)
 {
     Proj P[G];
     float ph[G];
     const SrcLds *SS[G];
 #pragma unroll
     for (int k = 0; k < G; ++k) {
-        P[k] = make_proj(Ss, du, dv, hd[K0 + k + 1], ak[K0 + k], bk[K0 + k]);
+        const bool on = k < U.n;
+        P[k] = make_proj(Ss, U.du, U.dv, on ? U.d[k] : U.d[0], on ? U.a[k] : U.a[0], on ? U.b[k] : U.b[0]);
         SS[k] = &Ss;
     }
     // geometric term first: its depth gathers overlap the window pass
     float gt[G];
 #pragma unroll
     for (int k = 0; k < G; ++k)
-        gt[k] = pass == 1 ? c.geom_reg * fminf(geo_error(c, Ss, P[k], du, dv), c.geom_max) : 0.f;
-    ncc_cost_group<G>(c, SS, P, s_ref, lbase, R, ph, nullptr, hyp_ok);
+        gt[k] = pass == 1 ? c.geom_reg * fminf(geo_error(c, Ss, P[k], U.du, U.dv), c.geom_max) : 0.f;
+    ncc_cost_group<G>(c, SS, P, s_ref, U.lbase, U.R, ph, nullptr, hyp_ok);
 #pragma unroll
-    for (int k = 0; k < G; ++k) acc[K0 + k] += cnt * (pass == 1 ? ph[k] + gt[k] : ph[k]);
+    for (int k = 0; k < G; ++k) res[k] = pass == 1 ? ph[k] + gt[k] : ph[k];
 }
 
-// All candidate hypotheses 1 .. kNHyp-1 in groups of (at most) G.
-template <int G, int K0>
-__device__ __forceinline__ void eval_hyps(const PMConst &c, const SrcLds &Ss, float cnt, int pass,
-                                          float du, float dv, const float (&hd)[kNHyp],
-                                          const float (&ak)[kNHyp - 1], const float (&bk)[kNHyp - 1],
-                                          const float *s_ref, int lbase, const RefStats &R,
-                                          float (&acc)[kNHyp - 1], bool hyp_ok)
+__device__ __forceinline__ int lane_id() { return __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u)); }
+__device__ __forceinline__ int bits_below(unsigned long long m)
 {
-    if constexpr (K0 < kNHyp - 1) {
-        constexpr int g = (kNHyp - 1 - K0) < G ? (kNHyp - 1 - K0) : G;
-        eval_hyp_group<g, K0>(c, Ss, cnt, pass, du, dv, hd, ak, bk, s_ref, lbase, R, acc, hyp_ok);
-        eval_hyps<G, K0 + g>(c, Ss, cnt, pass, du, dv, hd, ak, bk, s_ref, lbase, R, acc, hyp_ok);
+    return __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
+}
+__device__ __forceinline__ int from_lane(int lane, int v) { return __builtin_amdgcn_ds_bpermute(lane << 2, v); }
+__device__ __forceinline__ float from_lane(int lane, float v)
+{
+    return __int_as_float(__builtin_amdgcn_ds_bpermute(lane << 2, __float_as_int(v)));
+}
+
+// Drop the planes whose partial sum has reached `bound`, keeping the order of
+// the others; ids holds the candidates' indices, four bits each.
+__device__ __forceinline__ void drop_hyps(float (&d)[kGroupH], float (&a)[kGroupH], float (&b)[kGroupH],
+                                          float (&acc)[kGroupH], uint32_t &ids, int &live, int l, float bound)
+{
+#pragma unroll
+    for (int k = kGroupH - 1; k >= 0; --k) {
+        const bool out = k < l && acc[k] >= bound;
+        if (__ballot(out) == 0ull) continue;
+#pragma unroll
+        for (int j = k; j + 1 < kGroupH; ++j) {
+            d[j] = out ? d[j + 1] : d[j];
+            a[j] = out ? a[j + 1] : a[j];
+            b[j] = out ? b[j + 1] : b[j];
+            acc[j] = out ? acc[j + 1] : acc[j];
+        }
+        const uint32_t lo = (1u << (4 * k)) - 1u;
+        ids = out ? (ids & lo) | ((ids >> 4) & ~lo) : ids;
+        live -= out ? 1 : 0;
     }
 }
 
@@ -903,13 +958,20 @@ __device__ __forceinline__ void halfstep_tile(const ViewDesc &V, const Tile &t, 
         // every candidate within the depth and slope bounds of the tile's
         // `inner` sources (|a| = |n0 / n2| <= amax checked without dividing,
         // with a margin for the division's rounding)
-        bool hyp_ok = true;
+        // wide_ok: the same of every lane of the wave with the wider depth
+        // range of `linear`, and every source `linear`
+        bool hyp_ok = true, wide_ok = true;
         {
             const float amx = 0.999f * slope_bound(c), dlo = hyp_depth_lo(V), dhi = hyp_depth_hi(V);
+            const float more = kLinearRange * range;
 #pragma unroll
-            for (int k = 0; k < kNHyp; ++k)
-                hyp_ok = hyp_ok && hd[k] >= dlo && hd[k] <= dhi && hn2[k] > 0.f &&
-                         fabsf(hn0[k]) <= amx * hn2[k] && fabsf(hn1[k]) <= amx * hn2[k];
+            for (int k = 0; k < kNHyp; ++k) {
+                const bool slope = hn2[k] > 0.f && fabsf(hn0[k]) <= amx * hn2[k] && fabsf(hn1[k]) <= amx * hn2[k];
+                hyp_ok = hyp_ok && slope && hd[k] >= dlo && hd[k] <= dhi;
+                wide_ok = wide_ok && slope && hd[k] >= dlo - more && hd[k] <= dhi + more;
+            }
+            for (int s = 0; s < S; ++s) wide_ok = wide_ok && s_src[s].linear != 0;
+            wide_ok = __ballot(!wide_ok) == 0ull;
         }
 
         // ---- view selection on the current hypothesis --------------------
@@ -1070,33 +1132,142 @@ __device__ __forceinline__ void halfstep_tile(const ViewDesc &V, const Tile &t, 
         }
 
         // ---- evaluate the other seven hypotheses -------------------------
-        // One pass over the window per sampled source evaluates all seven.
-        // Sources are visited in ascending order by the whole wave (a lane
-        // that did not draw source s is masked off), so every gather of a
-        // pass reads one source image; each lane still accumulates its drawn
-        // sources in ascending order.
-        float ak[kNHyp - 1], bk[kNHyp - 1], acc[kNHyp - 1];
-#pragma unroll
-        for (int k = 0; k < kNHyp - 1; ++k) {
-            ak[k] = -hn0[k + 1] / hn2[k + 1];
-            bk[k] = -hn1[k + 1] / hn2[k + 1];
-            acc[k] = 0.f;
-        }
-        for (int s = 0; s < S; ++s) {
-            const uint32_t e = s_list[s * kThreads + tid];
-            if (e == 0u) continue;
-            const SrcLds &Ss = s_src[s];
-            const float cnt = (float)e;
-            eval_hyps<kGroupH, 0>(c, Ss, cnt, pass, du, dv, hd, ak, bk, s_ref, lbase, R, acc, hyp_ok);
-        }
-        my_ncc += (kNHyp - 1) * nlist;
-        if (pass == 1) my_geo += (kNHyp - 1) * nlist;
-        float best_c = acc0 / wsum;
+        // One pass over the window per sampled source evaluates up to
+        // kGroupH of them: first the four propagated planes, then the random
+        // and the perturbed ones.  Sources are visited in ascending order by
+        // the whole wave (a lane that did not draw source s is masked off),
+        // so every gather of a pass reads one source image; each lane still
+        // accumulates its drawn sources in ascending order.
+        // Costs are not negative, so a sum never falls: a candidate whose
+        // partial sum has reached the best complete one cannot win (division
+        // by wsum keeps the order, and the lower index wins ties) and leaves
+        // the lane's list.  A pass is as wide as the longest list of its
+        // lanes, and ends with the last list; where idle lanes (source not
+        // drawn, list empty) can take the parts of longer lists it is
+        // narrower still.  Bound as before by the texture data path (95 %
+        // busy) with VALU issue (87 -> 80 %) behind: evaluations -22 %, VALU
+        // instructions -14 % (10 views of 1024^2, 8 sources, step 2) and
+        // -25 % (4096^2, 20 sources).  Per half-step: 10.2 -> 9.6 ms and
+        // 32.2 -> 28.1 ms; one 1024^2 view at step 1 3.52 -> 3.21 ms; 2560^2
+        // with 16 sources, geometric 32.6 -> 28.6 ms.  Leaving early without
+        // the packing gave a third to a half of that.
+        const bool prune = wide_ok && (pass == 0 || (c.geom_reg >= 0.f && c.geom_max >= 0.f));
+        const bool spread = prune && __ballot(1) == ~0ull;
+        // one set of bounds for the wave, whichever lane takes a plane
+        const bool hyp_in = prune ? __ballot(!hyp_ok) == 0ull : hyp_ok;
+        float best_s = acc0, best_c = acc0 / wsum;
         int best = 0;
+#pragma unroll 1
+        for (int part = 0; part < 2; ++part) {
+            float d[kGroupH], a[kGroupH], b[kGroupH], acc[kGroupH];
 #pragma unroll
-        for (int k = 0; k < kNHyp - 1; ++k) {
-            const float ck = acc[k] / wsum;
-            if (ck < best_c) { best_c = ck; best = k + 1; }
+            for (int k = 0; k < kGroupH; ++k) {
+                const int k1 = k + 1, k2 = k + 5 < kNHyp ? k + 5 : kNHyp - 1;
+                const float n0 = part ? hn0[k2] : hn0[k1], n1 = part ? hn1[k2] : hn1[k1],
+                            n2 = part ? hn2[k2] : hn2[k1];
+                d[k] = part ? hd[k2] : hd[k1];
+                a[k] = -n0 / n2;
+                b[k] = -n1 / n2;
+                acc[k] = 0.f;
+            }
+            uint32_t ids = part ? 0x765u : 0x4321u;
+            int live = part ? kNHyp - 5 : kGroupH;
+            const float bound = prune ? best_s : INFINITY;
+            for (int s = 0; s < S; ++s) {
+                const uint32_t e = s_list[s * kThreads + tid];
+                const int l = e ? live : 0;
+                const unsigned long long m1 = __ballot(l > 0), m2 = __ballot(l > 1), m3 = __ballot(l > 2),
+                                         m4 = __ballot(l > 3);
+                if (m1 == 0ull) continue;
+                const SrcLds &Ss = s_src[s];
+                my_ncc += l;
+                if (pass == 1) my_geo += l;
+                const int n1 = __popcll(m1), n2 = __popcll(m2), n3 = __popcll(m3), n4 = __popcll(m4);
+                int G = n4 ? 4 : n3 ? 3 : n2 ? 2 : 1;
+                // A narrower pass whose units (n planes of a pixel make
+                // ceil(n / G) of them) fit the wave, idle lanes taking the
+                // parts beyond the first.
+                int gp = G;
+                if (spread) gp = n1 + n2 + n3 + n4 <= 64 ? 1 : n1 + n3 <= 64 ? 2 : n1 + n4 <= 64 ? 3 : 4;
+                const bool packed = gp < G;
+                G = packed ? gp : G;
+                Unit U;
+                U.du = du; U.dv = dv; U.lbase = lbase; U.n = l; U.R = R;
+#pragma unroll
+                for (int k = 0; k < kGroupH; ++k) { U.d[k] = d[k]; U.a[k] = a[k]; U.b[k] = b[k]; }
+                int to[kGroupH] = {0, 0, 0, 0};      // lane of part p of this lane's planes
+                if (packed) {
+                    const int lane = lane_id();
+                    int src = lane, part = 0, units = 0;
+#pragma unroll
+                    for (int q = 0; q < kGroupH; ++q) {
+                        if (q * G >= kGroupH) break;
+                        const unsigned long long mq = __ballot(l > q * G);
+                        const int nq = __popcll(mq), r = bits_below(mq);
+                        to[q] = units + r;
+                        // every lane sends, the ones without a part to the
+                        // lanes no part goes to
+                        const int dst = l > q * G ? to[q] : (units + nq + lane - r) & 63;
+                        const int got = __builtin_amdgcn_ds_permute(dst << 2, lane);
+                        if (lane >= units && lane < units + nq) { src = got; part = q; }
+                        units += nq;
+                    }
+                    const int h0 = part * G;
+                    const int ul = from_lane(src, l);
+                    U.n = lane < units ? ul - h0 : 0;
+                    const int txy = from_lane(src, tx | (ty << 8));
+                    const int ux = txy & 255, uy = txy >> 8;
+                    U.du = (float)(ux - T::W / 2);
+                    U.dv = (float)(uy - T::H / 2);
+                    U.lbase = (uy + kMaxRadius) * T::LW + ux + kMaxRadius;
+                    U.R.rc = s_ref[U.lbase];
+                    U.R.inv_sw = from_lane(src, R.inv_sw);
+                    U.R.mr = from_lane(src, R.mr);
+                    U.R.var_r = from_lane(src, R.var_r);
+                    U.R.wt = wtab ? s_w + (tid - lane + src) : nullptr;
+                    float fd[kGroupH], fa[kGroupH], fb[kGroupH];
+#pragma unroll
+                    for (int k = 0; k < kGroupH; ++k) {
+                        fd[k] = from_lane(src, d[k]); fa[k] = from_lane(src, a[k]); fb[k] = from_lane(src, b[k]);
+                    }
+#pragma unroll
+                    for (int k = 0; k < kGroupH - 1; ++k) {
+                        const int h = h0 + k;
+                        U.d[k] = h == 0 ? fd[0] : h == 1 ? fd[1] : h == 2 ? fd[2] : fd[3];
+                        U.a[k] = h == 0 ? fa[0] : h == 1 ? fa[1] : h == 2 ? fa[2] : fa[3];
+                        U.b[k] = h == 0 ? fb[0] : h == 1 ? fb[1] : h == 2 ? fb[2] : fb[3];
+                    }
+                }
+                float res[kGroupH] = {0.f, 0.f, 0.f, 0.f};
+                if (U.n > 0) {
+                    if (G == 4) eval_unit<4>(c, Ss, pass, U, s_ref, res, hyp_in);
+                    else if (G == 3) eval_unit<3>(c, Ss, pass, U, s_ref, res, hyp_in);
+                    else if (G == 2) eval_unit<2>(c, Ss, pass, U, s_ref, res, hyp_in);
+                    else eval_unit<1>(c, Ss, pass, U, s_ref, res, hyp_in);
+                }
+                const float cnt = (float)e;
+#pragma unroll
+                for (int k = 0; k < kGroupH; ++k) {
+                    float r = res[k];
+                    if (packed) {                    // plane k is slot k % G of part k / G
+                        const int q = G == 1 ? k : G == 2 ? k >> 1 : k / 3, j = k - q * G;
+                        r = from_lane((q == 0 ? to[0] : q == 1 ? to[1] : q == 2 ? to[2] : to[3]) & 63,
+                                      j == 0 ? res[0] : j == 1 ? res[1] : res[2]);
+                    }
+                    const float t = acc[k] + cnt * r;
+                    acc[k] = k < l ? t : acc[k];
+                }
+                if (s + 1 < S) drop_hyps(d, a, b, acc, ids, live, l, bound);
+            }
+#pragma unroll
+            for (int k = 0; k < kGroupH; ++k) {
+                const float ck = acc[k] / wsum;
+                if (k < live && ck < best_c) {
+                    best_c = ck;
+                    best_s = acc[k];
+                    best = (int)((ids >> (4 * k)) & 15u);
+                }
+            }
         }
         const float bd = pick8(best, hd[0], hd[1], hd[2], hd[3], hd[4], hd[5], hd[6], hd[7]);
         const float b0n = pick8(best, hn0[0], hn0[1], hn0[2], hn0[3], hn0[4], hn0[5], hn0[6], hn0[7]);
