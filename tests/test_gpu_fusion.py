@@ -133,6 +133,36 @@ def test_fuse_dsm_odd_grids_bit_exact(ctx, tiny, shape):
         assert any(np.isfinite(v).any() for v in views)
 
 
+@pytest.mark.parametrize("n_views,cell,holes", [(1, 0.5, 0.5), (3, 0.23, 0.3), (8, 0.23, 0.9), (9, 0.3, 0.1),
+                                                (24, 0.5, 0.6), (25, 1.1, 0.7), (40, 0.3, 0.2), (41, 0.5, 0.0),
+                                                (56, 0.5, 0.95), (64, 0.5, 0.4)])
+def test_fuse_stack_sizes_and_densities_bit_exact(ctx, n_views, cell, holes):
+    """View counts on both sides of the stack kernel's register counts
+    (multiples of 8 up to 64), cells finer and coarser than the pixels (empty
+    cells with few and with many neighbours) and sparse maps (windows with
+    some and with no values), with repeated heights."""
+    rng = np.random.default_rng(n_views)
+    W, H = 71, 37
+    inv = np.array([[0.5, 0, 0.25, 0], [0, -0.5, -0.25, 0], [0, 0, 0, 1], [0, 0, 1, 0]], dtype=np.float64)
+    grid = (1.0, -1.0, cell, cell, int(33 / cell), int(16 / cell))
+    base = rng.normal(50, 10, (H, W))
+    ids, depths = [], []
+    for v in range(n_views):
+        d = np.round(base + rng.normal(0, 2, (H, W)), 1).astype(np.float32)
+        d[rng.random((H, W)) < holes] = 0.0
+        ctx.register_geometry(300 + v, W, H, np.eye(4))
+        ctx.set_depth_map(300 + v, d, kind=1)
+        ids.append(300 + v)
+        depths.append(d)
+    fused, pv = ctx.fuse_dsm(grid, ids, depth_kind=1, min_measurements=min(3, n_views),
+                             inv_proj_mats=np.stack([inv] * n_views), per_view=True)
+    views = np.stack([fo.view_dsm(d, inv, grid) for d in depths])
+    assert np.isfinite(views).any()
+    for v in range(n_views):
+        assert _same(pv[v], views[v]), v
+    assert _same(fused, fo.fuse(views, min(3, n_views)))
+
+
 def test_fuse_dsm_rejects_bad_arguments(ctx):
     from vissatsatellitestereo_amd._lib import VsmError
     with pytest.raises(VsmError):

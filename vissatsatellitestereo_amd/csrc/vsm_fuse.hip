@@ -224,20 +224,29 @@ __global__ void k_unpack_fused(const FusedPoint *__restrict__ s, long long n, do
     gray[t] = (uint8_t)min(o.gray, 255u);
 }
 
-// Small in-register sort (insertion) of up to 9 doubles/floats.
+__device__ __forceinline__ float lower(float a, float b) { return fminf(a, b); }
+__device__ __forceinline__ float upper(float a, float b) { return fmaxf(a, b); }
+__device__ __forceinline__ double lower(double a, double b) { return fmin(a, b); }
+__device__ __forceinline__ double upper(double a, double b) { return fmax(a, b); }
+
+// Batcher's odd-even merge sort of N registers (static indices only, any N;
+// values are finite or infinite, no NaN: min and max order them).
 template <typename T, int N>
-__device__ __forceinline__ void sort_small(T (&v)[N], int n)
+__device__ __forceinline__ void sort_net(T (&v)[N])
 {
 #pragma unroll
-    for (int i = 1; i < N; ++i) {
-        if (i < n) {
-            T x = v[i];
+    for (int p = 1; p < N; p <<= 1)
 #pragma unroll
-            for (int j = i - 1; j >= 0; --j) {
-                if (v[j] > x) { v[j + 1] = v[j]; v[j] = x; }
+        for (int k = p; k >= 1; k >>= 1)
+#pragma unroll
+            for (int i = 0; i + k < N; ++i) {
+                const int j = k % p;
+                if (i >= j && (i - j) % (2 * k) < k && i / (2 * p) == (i + k) / (2 * p)) {
+                    const T lo = lower(v[i], v[i + k]), hi = upper(v[i], v[i + k]);
+                    v[i] = lo;
+                    v[i + k] = hi;
+                }
             }
-        }
-    }
 }
 
 template <typename T, int N>
@@ -245,7 +254,7 @@ __device__ __forceinline__ T median_sorted(const T (&v)[N], int n)
 {
     T lo = v[0], hi = v[0];
 #pragma unroll
-    for (int i = 0; i < N; ++i) {
+    for (int i = 0; i <= N / 2; ++i) {
         if (i == (n - 1) / 2) lo = v[i];
         if (i == n / 2) hi = v[i];
     }
@@ -277,138 +286,263 @@ __global__ void k_decode_fill(const unsigned long long *__restrict__ cell_max, i
             n += kk ? 1 : 0;
         }
     if (n == 0) { dsm[i] = (OUT)NAN; return; }
-    sort_small<double, 9>(v, 9);
+    sort_net<double, 9>(v);
     dsm[i] = (OUT)median_sorted<double, 9>(v, n);
 }
 
-// 3x3 median, replicated border, NaN excluded, all-NaN -> NaN.
-__global__ void k_median3(const float *__restrict__ in, int e_size, int n_size,
-                          float *__restrict__ out)
+// min, middle, max of three values (no NaN).
+__device__ __forceinline__ void sort3(float &a, float &b, float &c)
 {
-    const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= (long long)e_size * n_size) return;
-    const int r = (int)(i / e_size), c = (int)(i - (long long)r * e_size);
+    const float lo = __builtin_amdgcn_fmed3f(a, b, -INFINITY), hi = __builtin_amdgcn_fmed3f(a, b, INFINITY);
+    a = __builtin_amdgcn_fmed3f(lo, c, -INFINITY);
+    b = __builtin_amdgcn_fmed3f(lo, hi, c);
+    c = __builtin_amdgcn_fmed3f(hi, c, INFINITY);
+}
+
+// 3x3 medians of R cells in a column from the R + 2 rows of three values
+// around them, for the windows without NaN: each row is sorted once and serves
+// the three windows it is in, whose median is the middle of (largest of the
+// lowest, middle of the middle, lowest of the largest).  Bit r of the result:
+// window r holds a NaN and takes median_of_window.
+template <int R>
+__device__ __forceinline__ uint32_t column_medians(const float (&w)[R + 2][3], float (&out)[R])
+{
+    float lo[R + 2], mi[R + 2], hi[R + 2];
+    uint32_t nan = 0u;
+#pragma unroll
+    for (int r = 0; r < R + 2; ++r) {
+        lo[r] = w[r][0]; mi[r] = w[r][1]; hi[r] = w[r][2];
+        if (__builtin_isunordered(w[r][0], w[r][1]) || w[r][2] != w[r][2]) nan |= 7u << r;   // windows r - 2 .. r, shifted by 2
+        sort3(lo[r], mi[r], hi[r]);
+    }
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+        const float a = __builtin_amdgcn_fmed3f(__builtin_amdgcn_fmed3f(lo[r], lo[r + 1], INFINITY), lo[r + 2], INFINITY);
+        const float b = __builtin_amdgcn_fmed3f(mi[r], mi[r + 1], mi[r + 2]);
+        const float c = __builtin_amdgcn_fmed3f(__builtin_amdgcn_fmed3f(hi[r], hi[r + 1], -INFINITY), hi[r + 2], -INFINITY);
+        out[r] = __builtin_amdgcn_fmed3f(a, b, c);
+    }
+    return (nan >> 2) & ((1u << R) - 1u);
+}
+
+// Median of nine values: NaN excluded, even count -> mean of the two middle
+// values, all NaN -> NaN.
+__device__ __forceinline__ float median_of_window(const float (&x)[9])
+{
     float v[9];
     int n = 0;
 #pragma unroll
-    for (int dr = -1; dr <= 1; ++dr)
+    for (int k = 0; k < 9; ++k) {
+        v[k] = x[k] == x[k] ? x[k] : INFINITY;
+        n += x[k] == x[k] ? 1 : 0;
+    }
+    if (n == 0) return NAN;
+    sort_net<float, 9>(v);
+    return median_sorted<float, 9>(v, n);
+}
+
+// 3x3 median, replicated border, NaN excluded, all-NaN -> NaN.  A thread
+// takes kMedRows cells of a column (6554^2 cells: 345 -> 112 us).
+constexpr int kMedRows = 4;
+
+__global__ __launch_bounds__(256) void k_median3(const float *__restrict__ in, int e_size, int n_size,
+                                                 float *__restrict__ out)
+{
+    const unsigned int across = (e_size + 63) / 64;      // one-dimensional grid: any number of rows
+    const int c = (int)(blockIdx.x % across) * 64 + (threadIdx.x & 63);
+    const int r0 = ((int)(blockIdx.x / across) * 4 + (threadIdx.x >> 6)) * kMedRows;
+    if (c >= e_size || r0 >= n_size) return;
+    float w[kMedRows + 2][3], m[kMedRows];
+#pragma unroll
+    for (int r = 0; r < kMedRows + 2; ++r)
 #pragma unroll
         for (int dc = -1; dc <= 1; ++dc) {
-            const int rr = min(max(r + dr, 0), n_size - 1), cc = min(max(c + dc, 0), e_size - 1);
-            const float x = in[(size_t)rr * e_size + cc];
-            const int slot = (dr + 1) * 3 + (dc + 1);
-            v[slot] = x == x ? x : INFINITY;
-            n += x == x ? 1 : 0;
+            const int rr = min(max(r0 - 1 + r, 0), n_size - 1), cc = min(max(c + dc, 0), e_size - 1);
+            w[r][dc + 1] = in[(size_t)rr * e_size + cc];
         }
-    if (n == 0) { out[i] = NAN; return; }
-    sort_small<float, 9>(v, 9);
-    out[i] = median_sorted<float, 9>(v, n);
+    const uint32_t nan = column_medians<kMedRows>(w, m);
+#pragma unroll
+    for (int r = 0; r < kMedRows; ++r) {
+        if (!(nan >> r & 1u)) continue;
+        const float x[9] = {w[r][0], w[r][1], w[r][2], w[r + 1][0], w[r + 1][1], w[r + 1][2],
+                            w[r + 2][0], w[r + 2][1], w[r + 2][2]};
+        m[r] = median_of_window(x);
+    }
+#pragma unroll
+    for (int r = 0; r < kMedRows; ++r)
+        if (r0 + r < n_size) out[(size_t)(r0 + r) * e_size + c] = m[r];
 }
 
 // Per-view DSM in one pass over a tile of kVT_W x kVT_H cells: decode the
 // cell keys, fill each empty cell with the median of its non-empty 3x3
 // neighbours (the unfilled keys, as k_decode_fill), then the 3x3 median of
 // the filled values (replicated border, NaN excluded, as k_median3) into
-// `out`.  The keys of the tile and a 2-cell halo are staged in LDS, the
-// filled values of the tile and a 1-cell halo (at border-clamped positions)
-// too, so each key is read once per tile instead of by three kernels.  The
-// tile's cells of `clear` (the other key grid, which the next view
-// rasterises into) are zeroed; `keys` and `clear` must differ, since other
-// tiles read this tile's keys as their halo.
+// `out`.  The heights of the tile and a 2-cell halo and the filled values of
+// the tile and a 1-cell halo sit in LDS, at the same indices, so each key is
+// read and decoded once per tile instead of by three kernels.  The tile's
+// cells of `clear` (the other key grid, which the next view rasterises into)
+// are zeroed; `keys` and `clear` must differ, since other tiles read this
+// tile's keys as their halo.
+//
+// Bound by VALU issue, not by the 20 bytes a cell moves, so the rare work is
+// listed and done by full waves: a wave of the tile nearly always holds an
+// empty cell, and often a window with a NaN.  Where no lane of a wave has more
+// than five neighbours (a grid finer than the pixels) the three largest of
+// them hold the median, else all nine are sorted.  The medians share their
+// rows' sorts (column_medians).  6554^2 cells of 0.3 m from 4096^2 pixels of
+// 0.6 m: 789 -> 420 us.
 constexpr int kVT_W = 64, kVT_H = 16;
+
+__device__ __forceinline__ double min_f64(double a, double b)
+{
+    double r;
+    asm("v_min_f64 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));   // fmin would quieten its operands first
+    return r;
+}
+__device__ __forceinline__ double max_f64(double a, double b)
+{
+    double r;
+    asm("v_max_f64 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+    return r;
+}
+
+// Median of the n heights among v (the others are -inf), n > 0.  few: no lane
+// of the wave has more than five.
+__device__ __forceinline__ double median_of_heights(double (&v)[9], int n, bool few)
+{
+    double lo, hi;                             // the two middle ones (the same for an odd count)
+    if (few) {
+        double a = max_f64(v[0], v[1]), b = min_f64(v[0], v[1]), c = min_f64(b, v[2]);
+        const double t = max_f64(b, v[2]);     // a >= b >= c: the largest so far
+        b = min_f64(a, t);
+        a = max_f64(a, t);
+#pragma unroll
+        for (int k = 3; k < 9; ++k) {
+            const double p = min_f64(a, v[k]), q = min_f64(b, p);
+            a = max_f64(a, v[k]);
+            b = max_f64(b, p);
+            c = max_f64(c, q);
+        }
+        // the n/2-th and (n-1)/2-th of n ascending, counted from the top
+        hi = n >= 5 ? c : n >= 3 ? b : a;
+        lo = n >= 4 ? c : n >= 2 ? b : a;
+    } else {
+        sort_net<double, 9>(v);                // the n heights are the last n
+        lo = hi = v[8];
+#pragma unroll
+        for (int k = 4; k < 8; ++k) {
+            if (k == 9 - n + (n - 1) / 2) lo = v[k];
+            if (k == 9 - n + n / 2) hi = v[k];
+        }
+    }
+    return (n & 1) ? hi : 0.5 * (lo + hi);
+}
 
 __global__ void __launch_bounds__(256) k_view_dsm(const unsigned long long *__restrict__ keys,
                                                   unsigned long long *__restrict__ clear, int e_size,
                                                   int n_size, float *__restrict__ out)
 {
-    constexpr int KW = kVT_W + 4, KH = kVT_H + 4, FW = kVT_W + 2, FH = kVT_H + 2;
-    __shared__ unsigned long long sk[KH * KW];
-    __shared__ float sf[FH * FW];
+    constexpr int KW = kVT_W + 4, KH = kVT_H + 4;
+    constexpr double kEmpty = -(double)INFINITY;
+    __shared__ double sk[KH * KW];             // heights, -inf where empty
+    __shared__ float sf[KH * KW];              // filled values, NaN where there is none
+    __shared__ unsigned short list[KH * KW];   // empty cells, then windows with a NaN
+    __shared__ int n_holes, n_windows;
     const int c0 = blockIdx.x * kVT_W, r0 = blockIdx.y * kVT_H;
-    for (int t = threadIdx.x; t < KH * KW; t += blockDim.x) {
+    if (threadIdx.x == 0) { n_holes = 0; n_windows = 0; }
+    __syncthreads();
+    for (int t = threadIdx.x; t < KH * KW; t += 256) {
         const int ky = t / KW, kx = t - ky * KW;
         const int r = r0 - 2 + ky, c = c0 - 2 + kx;
-        sk[t] = (r >= 0 && c >= 0 && r < n_size && c < e_size) ? keys[(size_t)r * e_size + c] : 0ull;
+        unsigned long long k = 0ull;
+        const bool inside = r >= 0 && c >= 0 && r < n_size && c < e_size;
+        if (inside) k = keys[(size_t)r * e_size + c];
+        const double z = k ? dec_f64(k) : kEmpty;
+        sk[t] = z;
+        if (k) sf[t] = (float)z;
+        else if (inside && ky > 0 && ky < KH - 1 && kx > 0 && kx < KW - 1)
+            list[atomicAdd(&n_holes, 1)] = (unsigned short)t;
     }
     __syncthreads();
-    for (int t = threadIdx.x; t < FH * FW; t += blockDim.x) {
-        const int fy = t / FW, fx = t - fy * FW;
-        // the filled value at the border-clamped position (the median below
-        // reads replicated borders)
-        const int rc = min(max(r0 - 1 + fy, 0), n_size - 1), cc = min(max(c0 - 1 + fx, 0), e_size - 1);
-        const int ky = rc - (r0 - 2), kx = cc - (c0 - 2);
-        const unsigned long long k = sk[ky * KW + kx];
-        float f;
-        if (k != 0ull) {
-            f = (float)dec_f64(k);
-        } else {
-            double v[9];
-            int n = 0;
-#pragma unroll
-            for (int dr = -1; dr <= 1; ++dr)
-#pragma unroll
-                for (int dc = -1; dc <= 1; ++dc) {
-                    const unsigned long long kk = sk[(ky + dr) * KW + kx + dc];
-                    const int slot = (dr + 1) * 3 + (dc + 1);
-                    v[slot] = kk ? dec_f64(kk) : (double)INFINITY;
-                    n += kk ? 1 : 0;
-                }
-            if (n == 0) {
-                f = NAN;
-            } else {
-                sort_small<double, 9>(v, 9);
-                f = (float)median_sorted<double, 9>(v, n);
-            }
-        }
-        sf[t] = f;
-    }
-    __syncthreads();
-    for (int t = threadIdx.x; t < kVT_W * kVT_H; t += blockDim.x) {
-        const int ty = t / kVT_W, tx = t - ty * kVT_W;
-        const int r = r0 + ty, c = c0 + tx;
-        if (r >= n_size || c >= e_size) continue;
-        float v[9];
+    for (int h = threadIdx.x; h < n_holes; h += 256) {
+        const int at = list[h];
+        double v[9];
         int n = 0;
 #pragma unroll
-        for (int dr = -1; dr <= 1; ++dr)
+        for (int k = 0; k < 9; ++k) {
+            v[k] = sk[at + (k / 3 - 1) * KW + k % 3 - 1];
+            n += v[k] != kEmpty ? 1 : 0;
+        }
+        const double z = median_of_heights(v, n, __ballot(n > 5) == 0ull);
+        sf[at] = n ? (float)z : NAN;
+    }
+    __syncthreads();
+    if (r0 == 0 || c0 == 0 || r0 + kVT_H >= n_size || c0 + kVT_W >= e_size) {
+        // the median reads replicated borders: the ring of cells just outside
+        for (int t = threadIdx.x; t < KH * KW; t += 256) {
+            const int ky = t / KW, kx = t - ky * KW;
+            const int r = r0 - 2 + ky, c = c0 - 2 + kx;
+            if (r < -1 || c < -1 || r > n_size || c > e_size || (r >= 0 && c >= 0 && r < n_size && c < e_size)) continue;
+            sf[t] = sf[(min(max(r, 0), n_size - 1) - r0 + 2) * KW + min(max(c, 0), e_size - 1) - c0 + 2];
+        }
+        __syncthreads();
+    }
+    constexpr int RT = kVT_H / 4;              // rows per thread
+    const int tx = threadIdx.x & 63, ty = (threadIdx.x >> 6) * RT;
+    const int c = c0 + tx;
+    if (c < e_size) {
+        float w[RT + 2][3], m[RT];
 #pragma unroll
-            for (int dc = -1; dc <= 1; ++dc) {
-                const float x = sf[(ty + 1 + dr) * FW + tx + 1 + dc];
-                const int slot = (dr + 1) * 3 + (dc + 1);
-                v[slot] = x == x ? x : INFINITY;
-                n += x == x ? 1 : 0;
-            }
-        const size_t i = (size_t)r * e_size + c;
-        clear[i] = 0ull;
-        if (n == 0) { out[i] = NAN; continue; }
-        sort_small<float, 9>(v, 9);
-        out[i] = median_sorted<float, 9>(v, n);
+        for (int r = 0; r < RT + 2; ++r)
+#pragma unroll
+            for (int k = 0; k < 3; ++k) w[r][k] = sf[(ty + 1 + r) * KW + tx + 1 + k];
+        const uint32_t nan = column_medians<RT>(w, m);
+#pragma unroll
+        for (int r = 0; r < RT; ++r) {
+            if (r0 + ty + r >= n_size) continue;
+            const size_t i = (size_t)(r0 + ty + r) * e_size + c;
+            clear[i] = 0ull;
+            if (nan >> r & 1u) list[atomicAdd(&n_windows, 1)] = (unsigned short)((ty + r) * kVT_W + tx);
+            else out[i] = m[r];
+        }
+    }
+    __syncthreads();
+    for (int h = threadIdx.x; h < n_windows; h += 256) {
+        const int t = list[h], ky = t / kVT_W, kx = t % kVT_W;
+        float x[9];
+#pragma unroll
+        for (int k = 0; k < 9; ++k) x[k] = sf[(ky + 1 + k / 3) * KW + kx + 1 + k % 3];
+        out[(size_t)(r0 + ky) * e_size + c0 + kx] = median_of_window(x);
     }
 }
 
-// Bitonic sort network over N registers (static indices only).
+// Sorts a sequence that falls and then rises (with +inf at its end): one
+// bitonic merge, the registers beyond N being +inf.
 template <int N>
-__device__ __forceinline__ void bitonic(float (&v)[N])
+__device__ __forceinline__ void merge_valley(float (&v)[N])
 {
+    constexpr int M = N <= 8 ? 8 : N <= 16 ? 16 : N <= 32 ? 32 : 64;
 #pragma unroll
-    for (int k = 2; k <= N; k <<= 1)
+    for (int j = M / 2; j > 0; j >>= 1)
 #pragma unroll
-        for (int j = k >> 1; j > 0; j >>= 1)
-#pragma unroll
-            for (int i = 0; i < N; ++i) {
-                const int l = i ^ j;
-                if (l > i) {
-                    // values are finite or +inf (no NaN): min/max order them
-                    const float a = v[i], b = v[l];
-                    const float lo = fminf(a, b), hi = fmaxf(a, b);
-                    v[i] = (i & k) == 0 ? lo : hi;
-                    v[l] = (i & k) == 0 ? hi : lo;
-                }
+        for (int i = 0; i < N; ++i) {
+            const int l = i ^ j;
+            if (l > i && l < N) {
+                const float lo = fminf(v[i], v[l]), hi = fmaxf(v[i], v[l]);
+                v[i] = lo;
+                v[l] = hi;
             }
+        }
 }
 
+// Cross-view fusion of a cell: median, median absolute deviation, mean of what
+// lies within it.  N is the view count rounded up to 8, so a 40-view stack
+// sorts 40 registers (305 comparators), not 64.  The deviations of the sorted
+// values fall and then rise, so their median takes a merge, not a second sort
+// (40 views of 6554^2 cells: 13.0 -> 3.3 ms with two 64-register bitonic sorts
+// before, 2.1 TB/s of the stack).
 template <int N>
-__global__ void k_fuse_stack(const float *__restrict__ stack, int nviews, long long ncell,
+__global__ __launch_bounds__(256) void k_fuse_stack(const float *__restrict__ stack, int nviews, long long ncell,
                              int min_measurements, float *__restrict__ out)
 {
     const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
@@ -426,11 +560,11 @@ __global__ void k_fuse_stack(const float *__restrict__ stack, int nviews, long l
     float s[N];
 #pragma unroll
     for (int k = 0; k < N; ++k) s[k] = v[k];
-    bitonic<N>(s);
+    sort_net<float, N>(s);
     const float med = median_sorted<float, N>(s, n);
 #pragma unroll
-    for (int k = 0; k < N; ++k) s[k] = v[k] == INFINITY ? INFINITY : fabsf(v[k] - med);
-    bitonic<N>(s);
+    for (int k = 0; k < N; ++k) s[k] = s[k] == INFINITY ? INFINITY : fabsf(s[k] - med);
+    merge_valley<N>(s);
     const float mad = median_sorted<float, N>(s, n);
     double acc = 0.0;
     int m = 0;
@@ -533,19 +667,28 @@ hipError_t launch_view_dsm(const unsigned long long *keys, unsigned long long *c
 
 hipError_t launch_median3(const float *in, int e_size, int n_size, float *out, hipStream_t st)
 {
-    k_median3<<<nblk((long long)e_size * n_size, 256), 256, 0, st>>>(in, e_size, n_size, out);
+    const unsigned int grid = nblk(e_size, 64) * nblk(n_size, 4 * kMedRows);
+    k_median3<<<grid, 256, 0, st>>>(in, e_size, n_size, out);
     return hipGetLastError();
 }
 
 hipError_t launch_fuse_stack(const float *stack, int nviews, long long ncell, int min_measurements,
                              float *out, hipStream_t st)
 {
-    const unsigned int b = nblk(ncell, 256);
-    if (nviews <= 8) k_fuse_stack<8><<<b, 256, 0, st>>>(stack, nviews, ncell, min_measurements, out);
-    else if (nviews <= 16) k_fuse_stack<16><<<b, 256, 0, st>>>(stack, nviews, ncell, min_measurements, out);
-    else if (nviews <= 32) k_fuse_stack<32><<<b, 256, 0, st>>>(stack, nviews, ncell, min_measurements, out);
-    else if (nviews <= 64) k_fuse_stack<64><<<b, 256, 0, st>>>(stack, nviews, ncell, min_measurements, out);
-    else return hipErrorInvalidValue;
+    if (nviews > 64) return hipErrorInvalidValue;
+    void (*fn)(const float *, int, long long, int, float *) = nullptr;
+    switch ((nviews + 7) / 8) {
+    case 0:
+    case 1: fn = k_fuse_stack<8>; break;
+    case 2: fn = k_fuse_stack<16>; break;
+    case 3: fn = k_fuse_stack<24>; break;
+    case 4: fn = k_fuse_stack<32>; break;
+    case 5: fn = k_fuse_stack<40>; break;
+    case 6: fn = k_fuse_stack<48>; break;
+    case 7: fn = k_fuse_stack<56>; break;
+    default: fn = k_fuse_stack<64>; break;
+    }
+    fn<<<nblk(ncell, 256), 256, 0, st>>>(stack, nviews, ncell, min_measurements, out);
     return hipGetLastError();
 }
 
