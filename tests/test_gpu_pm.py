@@ -525,6 +525,23 @@ def test_get_depth_map_round_trip(tiny):
         ctx.close()
 
 
+@pytest.mark.parametrize("w,h", [(511, 512), (512, 512), (513, 512), (1023, 2051), (3001, 2999)])
+def test_copies_to_host_are_whole(w, h):
+    """Maps on both sides of the size from which copies go through the pinned
+    ring, in pieces that do and do not divide them, and longer than the ring;
+    into fresh and into used memory, several copies in a row."""
+    ctx = _ctx()
+    rng = np.random.default_rng(w)
+    maps = [rng.random((h, w), dtype=np.float32) for _ in range(3)]
+    for i, m in enumerate(maps):
+        ctx.register_geometry(i + 1, w, h, np.eye(4))
+        ctx.set_depth_map(i + 1, m, kind=0)
+    for _ in range(2):
+        for i, m in enumerate(maps):
+            assert np.array_equal(ctx.get_depth_map(i + 1, kind=0), m)
+    ctx.close()
+
+
 def test_api_rejects_bad_input_and_stays_usable(tiny):
     """Invalid parameters and requests raise (nothing reaches a kernel) and
     leave the context as it was: a valid solve afterwards matches a fresh

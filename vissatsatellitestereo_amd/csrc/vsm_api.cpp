@@ -22,6 +22,7 @@
 #include <vector>
 
 #include "vissat_mvs.h"
+#include "vsm_copy.h"
 #include "vsm_device.h"
 #include "vsm_kernels.h"
 
@@ -57,6 +58,8 @@ struct Batch {
     vsm_params params;                      // snapshot at begin: every step and the filter use it
     std::vector<ViewState> views;
     std::vector<int> ref_ids;
+    std::vector<ViewDesc> hviews;           // sources of the uploads, kept until the stream is past them
+    std::vector<Tile> htiles;
     ViewDesc *dviews = nullptr;
     Tile *dtiles = nullptr;
     int ntiles = 0, maxs = 1;
@@ -130,6 +133,7 @@ struct vsm_ctx {
     // staged batched solves
     std::map<int, std::unique_ptr<Batch>> batches;
     int next_batch = 1;
+    CopyOut copier;                        // results to caller-owned host memory
 };
 
 namespace {
@@ -154,6 +158,28 @@ int fail(vsm_ctx *c, int code, const char *fmt, ...)
             return fail((ctx), VSM_EDEVICE, "%s failed: %s (%s:%d)", #expr, hipGetErrorString(e_), \
                         __FILE__, __LINE__);                                                    \
     } while (0)
+
+// Results to host memory: copy_out queues a copy behind the context's stream,
+// copies_done waits for the stream and for the data to be in place.  An entry
+// point that calls copy_out holds a CopyScope, so that no copy is under way
+// into the caller's memory when it returns early.
+hipError_t copy_out(vsm_ctx *c, void *dst, const void *src, size_t n)
+{
+    return c->copier.copy(dst, src, n, c->device, c->stream);
+}
+
+hipError_t copies_done(vsm_ctx *c)
+{
+    const hipError_t e = hipStreamSynchronize(c->stream);
+    const hipError_t w = c->copier.wait();
+    return e != hipSuccess ? e : w;
+}
+
+struct CopyScope {
+    explicit CopyScope(vsm_ctx *ctx) : c(ctx) {}
+    ~CopyScope() { (void)c->copier.wait(); }
+    vsm_ctx *c;
+};
 
 // Device memory: blocks freed by the library go to a per-context cache and
 // are reused by later allocations of up to the same size (all work runs in
@@ -614,40 +640,35 @@ int read_counters(vsm_ctx *c, const PMConst &pc)
     return VSM_OK;
 }
 
-int finalize_outputs(vsm_ctx *c, ViewState &vs, int pass, int ref_id, vsm_view_out *out,
-                     const uint32_t *d_mask)
+// dv: the view's descriptor on the device.
+int finalize_outputs(vsm_ctx *c, int pass, int ref_id, vsm_view_out *out, const uint32_t *d_mask,
+                     const ViewDesc *dv)
 {
     ImageRec &ref = c->images[ref_id];
     const size_t hw = (size_t)ref.W * ref.H;
-    ViewDesc *dv = nullptr;
     float *tmp = nullptr;
-    int rc = dalloc(c, &dv, 1);
-    if (!rc) rc = dalloc(c, &tmp, hw * 2);
-    if (rc) { dfree(c, dv); return rc; }
+    int rc = dalloc(c, &tmp, hw * 2);
+    if (rc) return rc;
     if ((!ref.depth[pass] && (rc = dalloc(c, &ref.depth[pass], hw))) ||
         (!ref.normal[pass] && (rc = dalloc(c, &ref.normal[pass], hw * 3)))) {
-        dfree(c, dv);
         dfree(c, tmp);
         return rc;
     }
-    HIPCHK(c, hipMemcpyAsync(dv, &vs.desc, sizeof(ViewDesc), hipMemcpyHostToDevice, c->stream));
     HIPCHK(c, launch_finalize(dv, 0, (int)hw, tmp, ref.normal[pass], tmp + hw, ref.depth[pass],
                               c->stream));
     if (pass == 0) ++ref.depth_ver;
     if (out && out->depth)
-        HIPCHK(c, hipMemcpyAsync(out->depth, tmp, hw * 4, hipMemcpyDeviceToHost, c->stream));
+        HIPCHK(c, copy_out(c, out->depth, tmp, hw * 4));
     if (out && out->normal)
-        HIPCHK(c, hipMemcpyAsync(out->normal, ref.normal[pass], hw * 12, hipMemcpyDeviceToHost,
-                                 c->stream));
+        HIPCHK(c, copy_out(c, out->normal, ref.normal[pass], hw * 12));
     if (out && out->cost)
-        HIPCHK(c, hipMemcpyAsync(out->cost, tmp + hw, hw * 4, hipMemcpyDeviceToHost, c->stream));
+        HIPCHK(c, copy_out(c, out->cost, tmp + hw, hw * 4));
     if (out && out->consistency) {
-        if (d_mask) HIPCHK(c, hipMemcpyAsync(out->consistency, d_mask, hw * 4, hipMemcpyDeviceToHost, c->stream));
+        if (d_mask) HIPCHK(c, copy_out(c, out->consistency, d_mask, hw * 4));
         else memset(out->consistency, 0, hw * 4);
     }
-    // dv and tmp go back to the cache; the copies above are ordered before
-    // any later use of them on the stream, and the caller synchronises
-    dfree(c, dv);
+    // tmp goes back to the cache; the copies above are ordered before any
+    // later use of it on the stream, and the caller waits for them
     dfree(c, tmp);
     return VSM_OK;
 }
@@ -693,8 +714,9 @@ int batch_begin(vsm_ctx *c, const vsm_view_req *reqs, int n, int pass, int use_g
         batch_release(c, b);
         return rc;
     }
-    std::vector<Tile> tiles;
-    std::vector<ViewDesc> hv(n);
+    std::vector<Tile> &tiles = b.htiles;
+    std::vector<ViewDesc> &hv = b.hviews;
+    hv.resize(n);
     for (int v = 0; v < n; ++v) {
         b.maxs = std::max(b.maxs, b.views[v].desc.n_src);
         tiles_for(b.views[v].desc, v, tiles, b.params.tile_width);
@@ -757,7 +779,6 @@ int batch_begin(vsm_ctx *c, const vsm_view_req *reqs, int n, int pass, int use_g
         }
         BEGINCHK(launch_init(b.dviews, b.dtiles, b.ntiles, pc, 0, b.params.tile_width, c->stream));
     }
-    BEGINCHK(hipStreamSynchronize(c->stream));
 #undef BEGINCHK
     return VSM_OK;
 }
@@ -813,8 +834,7 @@ int batch_step(vsm_ctx *c, Batch &b, int k)
         }
     }
     b.steps_done += m;
-    HIPCHK(c, hipStreamSynchronize(c->stream));
-    return read_counters(c, pc);
+    return read_counters(c, pc);               // waits for the half-steps
 }
 
 // Filter (when the batch's parameters ask for it) and outputs of every view.
@@ -822,6 +842,7 @@ int batch_finish(vsm_ctx *c, Batch &b, vsm_view_out *outs)
 {
     const int n = (int)b.views.size();
     const PMConst pc = make_const(b.params);
+    CopyScope scope(c);
     uint32_t *d_masks = nullptr;
     std::vector<size_t> mask_off(n, 0);
     int rc = VSM_OK;
@@ -853,9 +874,9 @@ int batch_finish(vsm_ctx *c, Batch &b, vsm_view_out *outs)
             rc = fail(c, VSM_EDEVICE, "hipStreamSynchronize failed: %s", hipGetErrorString(se));
     }
     for (int v = 0; v < n && !rc; ++v)
-        rc = finalize_outputs(c, b.views[v], b.pass, b.ref_ids[v], outs ? &outs[v] : nullptr,
-                              d_masks ? d_masks + mask_off[v] : nullptr);
-    const hipError_t se = hipStreamSynchronize(c->stream);
+        rc = finalize_outputs(c, b.pass, b.ref_ids[v], outs ? &outs[v] : nullptr,
+                              d_masks ? d_masks + mask_off[v] : nullptr, b.dviews + v);
+    const hipError_t se = copies_done(c);
     if (!rc && se != hipSuccess)
         rc = fail(c, VSM_EDEVICE, "hipStreamSynchronize failed: %s", hipGetErrorString(se));
     dfree(c, d_masks);
@@ -1081,8 +1102,9 @@ int vsm_get_depth_map(vsm_ctx *c, int32_t id, int32_t kind, float *depth, int32_
     if (w != r.W || h != r.H) return fail(c, VSM_EINVAL, "buffer %dx%d != image %dx%d", w, h, r.W, r.H);
     if (!r.depth[kind]) return fail(c, VSM_ENOENT, "image %d has no depth map of kind %d", id, kind);
     HIPCHK(c, hipSetDevice(c->device));
-    HIPCHK(c, hipMemcpyAsync(depth, r.depth[kind], (size_t)w * h * 4, hipMemcpyDeviceToHost, c->stream));
-    HIPCHK(c, hipStreamSynchronize(c->stream));
+    CopyScope scope(c);
+    HIPCHK(c, copy_out(c, depth, r.depth[kind], (size_t)w * h * 4));
+    HIPCHK(c, copies_done(c));
     return VSM_OK;
 }
 
@@ -1113,6 +1135,11 @@ int vsm_batch_begin(vsm_ctx *c, const vsm_view_req *reqs, int32_t n, int32_t pas
     auto b = std::make_unique<Batch>();
     const int rc = batch_begin(c, reqs, n, pass, use_graph, *b);
     if (rc) return rc;
+    const hipError_t e = hipStreamSynchronize(c->stream);
+    if (e != hipSuccess) {
+        batch_release(c, *b);
+        return fail(c, VSM_EDEVICE, "hipStreamSynchronize failed: %s", hipGetErrorString(e));
+    }
     const int id = c->next_batch++;
     c->batches[id] = std::move(b);
     *batch = id;
@@ -1390,10 +1417,10 @@ int vsm_fuse_dsm(vsm_ctx *c, const vsm_dsm_grid *grid, const int32_t *ids, int32
     }
     c->fuse_launches += 1;
     c->fuse_pixels += pixels;
-    HIPCHK(c, hipMemcpyAsync(dsm_out, fused, ncell * 4, hipMemcpyDeviceToHost, c->stream));
-    if (per_view_out)
-        HIPCHK(c, hipMemcpyAsync(per_view_out, stack, ncell * 4 * n, hipMemcpyDeviceToHost, c->stream));
-    HIPCHK(c, hipStreamSynchronize(c->stream));
+    CopyScope scope(c);
+    HIPCHK(c, copy_out(c, dsm_out, fused, ncell * 4));
+    if (per_view_out) HIPCHK(c, copy_out(c, per_view_out, stack, (size_t)ncell * 4 * n));
+    HIPCHK(c, copies_done(c));
     dfree(c, cells); dfree(c, stack); dfree(c, tmp); dfree(c, fused); dfree(c, mats);
     return VSM_OK;
 }
@@ -1478,6 +1505,7 @@ int vsm_fuse_points(vsm_ctx *c, const int32_t *ids, int32_t n, int32_t depth_kin
             return fail(c, VSM_EDEVICE, "%s failed: %s", #expr, hipGetErrorString(e_));        \
         }                                                                                       \
     } while (0)
+    CopyScope scope(c);
     F3CHK(hipMemcpyAsync(dviews, hv.data(), n * sizeof(Fuse3dView), hipMemcpyHostToDevice, c->stream));
     int64_t total = 0;
     for (int v = 0; v < n; ++v) {
@@ -1492,14 +1520,13 @@ int vsm_fuse_points(vsm_ctx *c, const int32_t *ids, int32_t n, int32_t depth_kin
         const int64_t put = std::min<int64_t>(room, ns);
         if (put > 0) {
             F3CHK(launch_unpack_fused(sel, put, dxyz, dnrm, dgray, c->stream));
-            F3CHK(hipMemcpyAsync(xyz + 3 * total, dxyz, put * 24, hipMemcpyDeviceToHost, c->stream));
-            if (normal)
-                F3CHK(hipMemcpyAsync(normal + 3 * total, dnrm, put * 12, hipMemcpyDeviceToHost, c->stream));
-            if (grey) F3CHK(hipMemcpyAsync(grey + total, dgray, put, hipMemcpyDeviceToHost, c->stream));
-            F3CHK(hipStreamSynchronize(c->stream));
+            F3CHK(copy_out(c, xyz + 3 * total, dxyz, put * 24));
+            if (normal) F3CHK(copy_out(c, normal + 3 * total, dnrm, put * 12));
+            if (grey) F3CHK(copy_out(c, grey + total, dgray, put));
         }
         total += ns;
     }
+    F3CHK(copies_done(c));
 #undef F3CHK
     cleanup();
     *count = total;
@@ -1526,8 +1553,9 @@ int vsm_proj_to_grid(vsm_ctx *c, const double *points, int64_t n, const vsm_dsm_
     HIPCHK(c, launch_fill_u64n(cells, ncell, 0ull, c->stream));
     HIPCHK(c, launch_rasterize_points(pts, n, g, cells, c->stream));
     HIPCHK(c, launch_decode_fill_f64(cells, g.e_size, g.n_size, out, c->stream));
-    HIPCHK(c, hipMemcpyAsync(dsm_out, out, ncell * 8, hipMemcpyDeviceToHost, c->stream));
-    HIPCHK(c, hipStreamSynchronize(c->stream));
+    CopyScope scope(c);
+    HIPCHK(c, copy_out(c, dsm_out, out, ncell * 8));
+    HIPCHK(c, copies_done(c));
     dfree(c, cells); dfree(c, out); dfree(c, pts);
     return VSM_OK;
 }
@@ -1632,9 +1660,9 @@ int vsm_enu_to_utm(vsm_ctx *c, const double *enu, int64_t n, double *out)
     if (rc) return rc;
     HIPCHK(c, hipMemcpyAsync(buf, enu, 24 * (size_t)n, hipMemcpyHostToDevice, c->stream));
     HIPCHK(c, launch_enu_to_utm(buf, n, c->geo, buf + 3 * (size_t)n, c->stream));
-    HIPCHK(c, hipMemcpyAsync(out, buf + 3 * (size_t)n, 24 * (size_t)n, hipMemcpyDeviceToHost,
-                             c->stream));
-    HIPCHK(c, hipStreamSynchronize(c->stream));
+    CopyScope scope(c);
+    HIPCHK(c, copy_out(c, out, buf + 3 * (size_t)n, 24 * (size_t)n));
+    HIPCHK(c, copies_done(c));
     dfree(c, buf);
     return VSM_OK;
 }
@@ -1651,8 +1679,9 @@ int vsm_median_blur3(vsm_ctx *c, const float *in, int32_t e_size, int32_t n_size
     if (rc) return rc;
     HIPCHK(c, hipMemcpyAsync(buf, in, nc * 4, hipMemcpyHostToDevice, c->stream));
     HIPCHK(c, launch_median3(buf, e_size, n_size, buf + nc, c->stream));
-    HIPCHK(c, hipMemcpyAsync(out, buf + nc, nc * 4, hipMemcpyDeviceToHost, c->stream));
-    HIPCHK(c, hipStreamSynchronize(c->stream));
+    CopyScope scope(c);
+    HIPCHK(c, copy_out(c, out, buf + nc, nc * 4));
+    HIPCHK(c, copies_done(c));
     dfree(c, buf);
     return VSM_OK;
 }
@@ -2088,12 +2117,12 @@ int vsm_poll(vsm_ctx *c, uint64_t ticket, vsm_view_out *out, int32_t *done)
         return e;
     }
     const size_t hw = (size_t)r.vs.desc.W * r.vs.desc.H;
-    if (out && out->depth) HIPCHK(c, hipMemcpyAsync(out->depth, r.out_depth, hw * 4, hipMemcpyDeviceToHost, c->stream));
-    if (out && out->normal) HIPCHK(c, hipMemcpyAsync(out->normal, r.out_normal, hw * 12, hipMemcpyDeviceToHost, c->stream));
-    if (out && out->cost) HIPCHK(c, hipMemcpyAsync(out->cost, r.out_cost, hw * 4, hipMemcpyDeviceToHost, c->stream));
-    if (out && out->consistency)
-        HIPCHK(c, hipMemcpyAsync(out->consistency, r.out_mask, hw * 4, hipMemcpyDeviceToHost, c->stream));
-    HIPCHK(c, hipStreamSynchronize(c->stream));
+    CopyScope scope(c);
+    if (out && out->depth) HIPCHK(c, copy_out(c, out->depth, r.out_depth, hw * 4));
+    if (out && out->normal) HIPCHK(c, copy_out(c, out->normal, r.out_normal, hw * 12));
+    if (out && out->cost) HIPCHK(c, copy_out(c, out->cost, r.out_cost, hw * 4));
+    if (out && out->consistency) HIPCHK(c, copy_out(c, out->consistency, r.out_mask, hw * 4));
+    HIPCHK(c, copies_done(c));
     dfree(c, r.out_depth);
     c->reqs.erase(it);
     return VSM_OK;

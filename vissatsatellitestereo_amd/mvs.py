@@ -113,9 +113,9 @@ class MvsContext:
         cap = int(capacity) if capacity is not None else sum(
             self.sizes[int(i)][0] * self.sizes[int(i)][1] for i in ids) // 2 + 1
         while True:
-            xyz = np.zeros((cap, 3), np.float64)
-            nrm = np.zeros((cap, 3), np.float32)
-            gry = np.zeros(cap, np.uint8)
+            xyz = np.empty((cap, 3), np.float64)
+            nrm = np.empty((cap, 3), np.float32)
+            gry = np.empty(cap, np.uint8)
             cnt = ctypes.c_int64()
             self._check(self.lib.vsm_fuse_points(
                 self.h, ids.ctypes.data_as(ctypes.POINTER(ctypes.c_int32)), len(ids), int(depth_kind),
@@ -128,7 +128,7 @@ class MvsContext:
     def get_depth_map(self, image_id, kind=1):
         """The depth map (kind 0 photometric, 1 geometric) held on the device."""
         h, w = self.sizes[int(image_id)]
-        out = np.zeros((h, w), np.float32)
+        out = np.empty((h, w), np.float32)
         self._check(self.lib.vsm_get_depth_map(self.h, int(image_id), int(kind), fptr(out), w, h))
         return out
 
@@ -158,16 +158,16 @@ class MvsContext:
             h, w = self.sizes[int(v["ref"])]
             res = {}
             if "depth" in want:
-                res["depth"] = np.zeros((h, w), np.float32)
+                res["depth"] = np.empty((h, w), np.float32)
                 outs[i].depth = fptr(res["depth"])
             if "normal" in want:
-                res["normal"] = np.zeros((h, w, 3), np.float32)
+                res["normal"] = np.empty((h, w, 3), np.float32)
                 outs[i].normal = fptr(res["normal"])
             if "cost" in want:
-                res["cost"] = np.zeros((h, w), np.float32)
+                res["cost"] = np.empty((h, w), np.float32)
                 outs[i].cost = fptr(res["cost"])
             if "consistency" in want:
-                res["consistency"] = np.zeros((h, w), np.uint32)
+                res["consistency"] = np.empty((h, w), np.uint32)
                 outs[i].consistency = u32ptr(res["consistency"])
             results.append(res)
         return outs, results
@@ -247,8 +247,8 @@ class MvsContext:
                  per_view=False):
         g = _lib.DsmGrid(*grid) if not isinstance(grid, _lib.DsmGrid) else grid
         ids = np.ascontiguousarray(image_ids, dtype=np.int32)
-        out = np.zeros((g.n_size, g.e_size), np.float32)
-        pv = np.zeros((len(ids), g.n_size, g.e_size), np.float32) if per_view else None
+        out = np.empty((g.n_size, g.e_size), np.float32)
+        pv = np.empty((len(ids), g.n_size, g.e_size), np.float32) if per_view else None
         mats = None
         if inv_proj_mats is not None:
             mats = np.ascontiguousarray(inv_proj_mats, dtype=np.float64).reshape(len(ids), 16)
@@ -262,7 +262,7 @@ class MvsContext:
     def proj_to_grid(self, points, grid):
         g = _lib.DsmGrid(*grid) if not isinstance(grid, _lib.DsmGrid) else grid
         pts = np.ascontiguousarray(points, dtype=np.float64).reshape(-1, 3)
-        out = np.zeros((g.n_size, g.e_size), np.float64)
+        out = np.empty((g.n_size, g.e_size), np.float64)
         self._check(self.lib.vsm_proj_to_grid(
             self.h, pts.ctypes.data_as(ctypes.POINTER(ctypes.c_double)) if len(pts) else None,
             len(pts), ctypes.byref(g), out.ctypes.data_as(ctypes.POINTER(ctypes.c_double))))
@@ -281,7 +281,7 @@ class MvsContext:
     def enu_to_utm(self, enu):
         """n x 3 local ENU -> n x 3 (easting, northing, altitude) on the device."""
         pts = np.ascontiguousarray(enu, dtype=np.float64).reshape(-1, 3)
-        out = np.zeros_like(pts)
+        out = np.empty_like(pts)
         if len(pts):
             self._check(self.lib.vsm_enu_to_utm(
                 self.h, pts.ctypes.data_as(ctypes.POINTER(ctypes.c_double)), len(pts),
@@ -290,7 +290,7 @@ class MvsContext:
 
     def median_blur3(self, img):
         a = np.ascontiguousarray(img, dtype=np.float32)
-        out = np.zeros_like(a)
+        out = np.empty_like(a)
         n_size, e_size = a.shape
         self._check(self.lib.vsm_median_blur3(self.h, fptr(a), e_size, n_size, fptr(out)))
         return out
@@ -318,16 +318,16 @@ class MvsContext:
         out = _lib.ViewOut()
         res = {}
         if "depth" in want:
-            res["depth"] = np.zeros((h, w), np.float32)
+            res["depth"] = np.empty((h, w), np.float32)
             out.depth = fptr(res["depth"])
         if "normal" in want:
-            res["normal"] = np.zeros((h, w, 3), np.float32)
+            res["normal"] = np.empty((h, w, 3), np.float32)
             out.normal = fptr(res["normal"])
         if "cost" in want:
-            res["cost"] = np.zeros((h, w), np.float32)
+            res["cost"] = np.empty((h, w), np.float32)
             out.cost = fptr(res["cost"])
         if "consistency" in want:
-            res["consistency"] = np.zeros((h, w), np.uint32)
+            res["consistency"] = np.empty((h, w), np.uint32)
             out.consistency = u32ptr(res["consistency"])
         done = ctypes.c_int32()
         self._check(self.lib.vsm_poll(self.h, ctypes.c_uint64(ticket), ctypes.byref(out),
