@@ -1198,20 +1198,24 @@ __device__ __forceinline__ void halfstep_tile(const ViewDesc &V, const Tile &t, 
                 int to[kGroupH] = {0, 0, 0, 0};      // lane of part p of this lane's planes
                 if (packed) {
                     const int lane = lane_id();
-                    int src = lane, part = 0, units = 0;
+                    int first = 0, units = 0;
 #pragma unroll
                     for (int q = 0; q < kGroupH; ++q) {
                         if (q * G >= kGroupH) break;
                         const unsigned long long mq = __ballot(l > q * G);
-                        const int nq = __popcll(mq), r = bits_below(mq);
-                        to[q] = units + r;
-                        // every lane sends, the ones without a part to the
-                        // lanes no part goes to
-                        const int dst = l > q * G ? to[q] : (units + nq + lane - r) & 63;
-                        const int got = __builtin_amdgcn_ds_permute(dst << 2, lane);
-                        if (lane >= units && lane < units + nq) { src = got; part = q; }
-                        units += nq;
+                        first += bits_below(mq);
+                        units += __popcll(mq);
                     }
+                    uint32_t *slot = s_list + s * kThreads + (tid - lane);
+#pragma unroll
+                    for (int q = 0; q < kGroupH; ++q) {
+                        if (q * G >= kGroupH) break;
+                        to[q] = first + q;
+                        if (l > q * G) slot[first + q] = (uint32_t)(lane | q << 6);
+                    }
+                    const int got = (int)slot[lane];
+                    slot[lane] = e;
+                    const int src = lane < units ? got & 63 : lane, part = lane < units ? got >> 6 : 0;
                     const int h0 = part * G;
                     const int ul = from_lane(src, l);
                     U.n = lane < units ? ul - h0 : 0;
@@ -1257,7 +1261,7 @@ __device__ __forceinline__ void halfstep_tile(const ViewDesc &V, const Tile &t, 
                     const float t = acc[k] + cnt * r;
                     acc[k] = k < l ? t : acc[k];
                 }
-                if (s + 1 < S) drop_hyps(d, a, b, acc, ids, live, l, bound);
+                if (S > 1) drop_hyps(d, a, b, acc, ids, live, l, bound);
             }
 #pragma unroll
             for (int k = 0; k < kGroupH; ++k) {
