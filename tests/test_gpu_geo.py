@@ -54,6 +54,27 @@ def test_enu_to_utm_bit_exact(ctx):
     ctx.set_geo_frame(None)
 
 
+def test_enu_to_utm_extremes_bit_exact(ctx):
+    """Points where the chain divides by small or large numbers or takes roots
+    of them: on the central meridian, on and near the axis and the Earth's
+    centre, far below and above, zero and non-finite offsets."""
+    from vissatsatellitestereo_amd import _lib
+    f = _lib.geo_frame(0.0, -81.0, 0.0, 17, 0)         # on the equator and the central meridian
+    rng = np.random.default_rng(17)
+    n = 50000
+    s = 10.0 ** rng.uniform(-12, 9, (n, 3)) * rng.choice([-1.0, 1.0], (n, 3))
+    s[rng.random((n, 3)) < 0.2] = 0.0
+    s[:200, 2] = -6378137.0 + 10.0 ** rng.uniform(-9, 3, 200)
+    s[200:210] = [[0, 0, 0], [0, 0, -6378137.0], [np.nan, 0, 0], [0, np.inf, 0], [0, 0, -np.inf],
+                  [1e160, 0, 0], [0, 1e160, 0], [0, 0, 1e200], [1e-300, 1e-300, 1e-300], [0, 6356752.0, -6378137.0]]
+    ctx.set_geo_frame(f)
+    g = ctx.enu_to_utm(s)
+    ctx.set_geo_frame(None)
+    o = go.enu_to_utm(f.as_array(), s)
+    assert np.isfinite(o[:, 0]).sum() > 1000
+    assert np.array_equal(g, o, equal_nan=True)
+
+
 def test_enu_to_utm_without_frame_fails(ctx):
     from vissatsatellitestereo_amd._lib import VsmError
     ctx.set_geo_frame(None)

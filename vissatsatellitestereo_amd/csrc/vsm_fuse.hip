@@ -54,15 +54,16 @@ __device__ __forceinline__ void cell_of(const DsmGridDev &g, double E, double N,
 // local_to_global + latlon_to_eastnorh (aggregate_2p5d_util.py:95-98) and the
 // cell value is the altitude.
 template <bool GEO>
-__global__ void k_rasterize_view(const float *__restrict__ depth, int W, int H,
+__global__ __launch_bounds__(256) void k_rasterize_view(const float *__restrict__ depth, int W, int H,
                                  const double *__restrict__ Mi, DsmGridDev g, vsm_geo_frame gf,
                                  unsigned long long *__restrict__ cell_max)
 {
-    const int p = blockIdx.x * blockDim.x + threadIdx.x;
-    if (p >= W * H) return;
-    const float d32 = depth[p];
+    // 64 x 4 pixels a workgroup: rows and columns without a division
+    const int px = blockIdx.x * 64 + (threadIdx.x & 63), py = blockIdx.y * 4 + (threadIdx.x >> 6);
+    if (px >= W || py >= H) return;
+    const float d32 = depth[(size_t)py * W + px];
     if (!(d32 > 0.f) || !isfinite(d32)) return;
-    const double col = (double)(p % W), row = (double)(p / W), d = (double)d32;
+    const double col = (double)px, row = (double)py, d = (double)d32;
     double X[4];
 #pragma unroll
     for (int i = 0; i < 4; ++i)
@@ -451,8 +452,8 @@ __global__ void __launch_bounds__(256) k_view_dsm(const unsigned long long *__re
     const int c0 = blockIdx.x * kVT_W, r0 = blockIdx.y * kVT_H;
     if (threadIdx.x == 0) { n_holes = 0; n_windows = 0; }
     __syncthreads();
-    for (int t = threadIdx.x; t < KH * KW; t += 256) {
-        const int ky = t / KW, kx = t - ky * KW;
+    auto load = [&](int ky, int kx) {
+        const int t = ky * KW + kx;
         const int r = r0 - 2 + ky, c = c0 - 2 + kx;
         unsigned long long k = 0ull;
         const bool inside = r >= 0 && c >= 0 && r < n_size && c < e_size;
@@ -462,7 +463,10 @@ __global__ void __launch_bounds__(256) k_view_dsm(const unsigned long long *__re
         if (k) sf[t] = (float)z;
         else if (inside && ky > 0 && ky < KH - 1 && kx > 0 && kx < KW - 1)
             list[atomicAdd(&n_holes, 1)] = (unsigned short)t;
-    }
+    };
+    // a wave takes 64 columns of every fourth row; the last four columns follow
+    for (int ky = threadIdx.x >> 6; ky < KH; ky += 4) load(ky, threadIdx.x & 63);
+    if (threadIdx.x < 4 * KH) load(threadIdx.x >> 2, 64 + (threadIdx.x & 3));
     __syncthreads();
     for (int h = threadIdx.x; h < n_holes; h += 256) {
         const int at = list[h];
@@ -592,12 +596,9 @@ hipError_t launch_rasterize_view(const float *depth, int W, int H, const double 
                                  DsmGridDev g, const vsm_geo_frame *geo,
                                  unsigned long long *cell_max, hipStream_t st)
 {
-    if (geo)
-        k_rasterize_view<true><<<nblk((long long)W * H, 256), 256, 0, st>>>(depth, W, H, invP4_dev,
-                                                                            g, *geo, cell_max);
-    else
-        k_rasterize_view<false><<<nblk((long long)W * H, 256), 256, 0, st>>>(
-            depth, W, H, invP4_dev, g, vsm_geo_frame{}, cell_max);
+    const dim3 grid((unsigned)((W + 63) / 64), (unsigned)((H + 3) / 4));
+    if (geo) k_rasterize_view<true><<<grid, 256, 0, st>>>(depth, W, H, invP4_dev, g, *geo, cell_max);
+    else k_rasterize_view<false><<<grid, 256, 0, st>>>(depth, W, H, invP4_dev, g, vsm_geo_frame{}, cell_max);
     return hipGetLastError();
 }
 

@@ -37,11 +37,44 @@
 namespace vsm {
 namespace geo {
 
+// Division and square root for the magnitudes of this chain (1e-20 .. 1e20):
+// correctly rounded like / and sqrt, without the scaling that the general ones
+// do against over- and underflow, and with the reciprocal shared by quotients
+// of one divisor.  Two Newton steps on the hardware's estimate, then the
+// residual correction of Markstein (1990, IBM J. Res. Dev. 34:111); the root by
+// Goldschmidt's iteration with two residual corrections (ibid.).  A zero, an
+// infinity or a NaN where the chain divides makes NaN, and the point is
+// dropped as it is by / and sqrt.  The conversion is bound by its FP64
+// instructions, of which these take out a quarter (16.8 Mpx rasterised on the
+// UTM grid: 520 -> 413 us).
+VSM_GEO_FN double reciprocal(double b)
+{
+    double y = __builtin_amdgcn_rcp(b);
+    y = fma(y, fma(-b, y, 1.0), y);
+    return fma(y, fma(-b, y, 1.0), y);
+}
+VSM_GEO_FN double quotient(double a, double b, double recip_b)
+{
+    const double q = a * recip_b;
+    return fma(fma(-b, q, a), recip_b, q);
+}
+VSM_GEO_FN double quotient(double a, double b) { return quotient(a, b, reciprocal(b)); }
+VSM_GEO_FN double root(double x)
+{
+    const double y = __builtin_amdgcn_rsq(x);
+    double g = x * y, h = 0.5 * y;
+    const double r = fma(-h, g, 0.5);
+    h = fma(h, r, h);
+    g = fma(g, r, g);
+    g = fma(fma(-g, g, x), h, g);
+    return fma(fma(-g, g, x), h, g);
+}
+
 VSM_GEO_FN void normalise(double x, double y, double &c, double &s)
 {
-    const double r = sqrt(x * x + y * y);
-    c = x / r;
-    s = y / r;
+    const double r = root(x * x + y * y), ir = reciprocal(r);
+    c = quotient(x, r, ir);
+    s = quotient(y, r, ir);
 }
 
 // atan(t) for |t| <= tan(pi/16): sum_k (-1)^k t^(2k+1) / (2k+1), k = 0..12.
@@ -72,16 +105,16 @@ VSM_GEO_FN double atan_any(double t)
     const bool neg = t < 0.0;
     double a = neg ? -t : t;
     const bool inv = a > 1.0;
-    if (inv) a = 1.0 / a;
-    a = a / (1.0 + sqrt(1.0 + a * a));
-    a = a / (1.0 + sqrt(1.0 + a * a));
+    if (inv) a = quotient(1.0, a);
+    a = quotient(a, 1.0 + root(1.0 + a * a));
+    a = quotient(a, 1.0 + root(1.0 + a * a));
     double r = 4.0 * atan_small(a);
     if (inv) r = kHalfPi - r;
     return neg ? -r : r;
 }
 
 // atan2(y, x) for x > 0.
-VSM_GEO_FN double atan2_xpos(double y, double x) { return atan_any(y / x); }
+VSM_GEO_FN double atan2_xpos(double y, double x) { return atan_any(quotient(y, x)); }
 
 // asinh(q) for |q| <= 0.25: sum_n (-1)^n (2n)! / (4^n (n!)^2 (2n+1)) q^(2n+1).
 VSM_GEO_FN double asinh_small(double q)
@@ -146,7 +179,7 @@ VSM_GEO_FN bool enu_to_utm(const vsm_geo_frame &f, double e, double n, double u,
     // longitude relative to the central meridian, as (cos, sin)
     const double xr = X * f.cm_cos + Y * f.cm_sin;
     const double yr = Y * f.cm_cos - X * f.cm_sin;
-    const double p = sqrt(X * X + Y * Y);
+    const double p = root(X * X + Y * Y);
     if (!(p > 0.0) || !(xr > 0.0)) return false;
     double cl, sl;
     normalise(xr, yr, cl, sl);
@@ -157,12 +190,12 @@ VSM_GEO_FN bool enu_to_utm(const vsm_geo_frame &f, double e, double n, double u,
         normalise(p - f.e2a * ((cb * cb) * cb), Z + f.ep2b * ((sb * sb) * sb), cp, sp);
         normalise(cp, f.one_minus_f * sp, cb, sb);
     }
-    alt = (p * cp + Z * sp) - f.a * sqrt(1.0 - f.e2 * (sp * sp));
+    alt = (p * cp + Z * sp) - f.a * root(1.0 - f.e2 * (sp * sp));
     // conformal latitude (Karney's tau')
-    const double tau = sp / cp;
+    const double tau = quotient(sp, cp);
     const double sig = sinh_small(f.e * atanh_small(f.e * sp));
-    const double taup = tau * sqrt(1.0 + sig * sig) - sig * sqrt(1.0 + tau * tau);
-    const double q = sl / sqrt(taup * taup + cl * cl);
+    const double taup = tau * root(1.0 + sig * sig) - sig * root(1.0 + tau * tau);
+    const double q = quotient(sl, root(taup * taup + cl * cl));
     if (!(q <= f.max_q && q >= -f.max_q)) return false;
     const double xip = atan2_xpos(taup, cl);
     const double etap = asinh_small(q);
@@ -170,7 +203,7 @@ VSM_GEO_FN bool enu_to_utm(const vsm_geo_frame &f, double e, double n, double u,
     double cx, sx;
     normalise(cl, taup, cx, sx);
     const double s2 = 2.0 * (sx * cx), c2 = cx * cx - sx * sx;
-    const double sh2 = 2.0 * (q * sqrt(1.0 + q * q)), ch2 = 1.0 + 2.0 * (q * q);
+    const double sh2 = 2.0 * (q * root(1.0 + q * q)), ch2 = 1.0 + 2.0 * (q * q);
     double sj[6], cj[6], shj[6], chj[6];
     sj[0] = s2; cj[0] = c2; shj[0] = sh2; chj[0] = ch2;
 #pragma unroll
