@@ -38,8 +38,8 @@ struct ImageRec {
     double Pinv[16];
     float *depth[2] = {nullptr, nullptr};   // photometric / geometric depth kept on device
     float *normal[2] = {nullptr, nullptr};  // camera-frame normals that go with depth[]
-    float4 *depth4 = nullptr;               // photometric depth, 2x2 neighbourhood per texel
-    uint64_t depth_ver = 0, depth4_ver = 0; // depth4 is current when the versions agree
+    float2 *depth2 = nullptr;               // photometric depth with the row below, (W + 1) x H texels
+    uint64_t depth_ver = 0, depth2_ver = 0; // depth2 is current when the versions agree
 };
 
 struct ViewState {
@@ -392,7 +392,7 @@ int build_geometry(vsm_ctx *c, const ImageRec &ref, const std::vector<const Imag
         V.src_w[s] = S.W;
         V.src_h[s] = S.H;
         V.src_pair[s] = (const uint8_t *)S.pair;
-        V.src_depth4[s] = nullptr;
+        V.src_depth2[s] = nullptr;
     }
     // Rotation of the reference camera from P[:3,:3] = K R.
     const double *A = ref.P4;
@@ -551,12 +551,12 @@ int prepare_view(vsm_ctx *c, const vsm_view_req &r, int pass, uint32_t view_id, 
                 return fail(c, VSM_EINVAL,
                             "geometric pass needs the photometric depth map of source image %d",
                             S.id);
-            if (!S.depth4 || S.depth4_ver != S.depth_ver) {
-                if (!S.depth4 && (rc = dalloc(c, &S.depth4, (size_t)S.W * S.H))) return rc;
-                HIPCHK(c, launch_pack_depth4(S.depth[0], S.W, S.H, S.depth4, c->stream));
-                S.depth4_ver = S.depth_ver;
+            if (!S.depth2 || S.depth2_ver != S.depth_ver) {
+                if (!S.depth2 && (rc = dalloc(c, &S.depth2, (size_t)(S.W + 1) * S.H))) return rc;
+                HIPCHK(c, launch_pack_depth2(S.depth[0], S.W, S.H, S.depth2, c->stream));
+                S.depth2_ver = S.depth_ver;
             }
-            V.src_depth4[s] = S.depth4;
+            V.src_depth2[s] = S.depth2;
         }
     }
     const size_t hw = (size_t)ref.W * ref.H;
@@ -1050,7 +1050,7 @@ int vsm_remove_image(vsm_ctx *c, int32_t id)
     dfree(c, r.depth[1]);
     dfree(c, r.normal[0]);
     dfree(c, r.normal[1]);
-    dfree(c, r.depth4);
+    dfree(c, r.depth2);
     c->images.erase(it);
     return VSM_OK;
 }
@@ -1724,7 +1724,8 @@ static size_t serve_footprint(vsm_ctx *c, const ServeReq &r, bool worst)
     if (r.pass == 1)
         for (int s : r.srcs) {
             const ImageRec &S = c->images.at(s);
-            if (worst || !S.depth4) b += (size_t)S.W * S.H * sizeof(float4);
+            // 16 bytes a pixel: twice what the texture takes, the admission rule as it was
+            if (worst || !S.depth2) b += (size_t)S.W * S.H * 16;
         }
     return b;
 }

@@ -31,7 +31,7 @@ hipError_t launch_finalize(const ViewDesc *views, int view, int npix, float *dep
                            float *cost, float *depth_keep, hipStream_t st);
 hipError_t launch_load_hyp(const ViewDesc *views, int view, int npix, const float *depth,
                            const float *normal, float cos_max_normal, hipStream_t st);
-hipError_t launch_pack_depth4(const float *depth, int W, int H, float4 *out, hipStream_t st);
+hipError_t launch_pack_depth2(const float *depth, int W, int H, float2 *out, hipStream_t st);
 hipError_t launch_pack_pair(const uint8_t *gray, int W, int H, uint16_t *pair, hipStream_t st);
 hipError_t launch_fill_u64(unsigned long long *p, int n, unsigned long long v, hipStream_t st);
 
