@@ -1714,7 +1714,8 @@ static size_t serve_footprint(vsm_ctx *c, const ServeReq &r, bool worst)
     if (r.pass == 1)
         for (int s : r.srcs) {
             const ImageRec &S = c->images.at(s);
-            // 16 bytes a pixel: twice what the texture takes, the admission rule as it was
+            // counted at 16 bytes a pixel, twice what the texture takes: a budget
+            // admits the mixes that it admitted with the wider texels
             if (worst || !S.depth2) b += (size_t)S.W * S.H * 16;
         }
     return b;

@@ -1150,9 +1150,9 @@ __device__ __forceinline__ void halfstep_tile(const ViewDesc &V, const Tile &t, 
         // narrower still.  Bound as before by the texture data path (95 %
         // busy) with VALU issue (87 -> 80 %) behind: evaluations -22 %, VALU
         // instructions -14 % (10 views of 1024^2, 8 sources, step 2) and
-        // -25 % (4096^2, 20 sources).  Per half-step: 10.2 -> 9.6 ms and
-        // 32.2 -> 28.1 ms; one 1024^2 view at step 1 3.52 -> 3.21 ms; 2560^2
-        // with 16 sources, geometric 32.6 -> 28.6 ms.  Leaving early without
+        // -25 % (4096^2, 20 sources).  Per half-step: 10.2 -> 9.4 ms and
+        // 32.2 -> 28.2 ms; one 1024^2 view at step 1 3.52 -> 3.21 ms; 2560^2
+        // with 16 sources, geometric 32.6 -> 28.3 ms.  Leaving early without
         // the packing gave a third to a half of that.
         const bool prune = wide_ok && (pass == 0 || (c.geom_reg >= 0.f && c.geom_max >= 0.f));
         const bool spread = prune && __ballot(1) == ~0ull;
