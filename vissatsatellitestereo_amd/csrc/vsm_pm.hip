@@ -826,6 +826,18 @@ __device__ __forceinline__ float from_lane(int lane, float v)
     return __int_as_float(__builtin_amdgcn_ds_bpermute(lane << 2, __float_as_int(v)));
 }
 
+// Orders the LDS accesses of a wave's lanes to each other: what any lane stored
+// before is what every lane loads after.  The lanes run in step and the LDS
+// takes their accesses in order, so this is no instruction; it keeps the
+// compiler, to which another lane's store is another thread's, from using a
+// value that it loaded or stored before for one that another lane has replaced.
+__device__ __forceinline__ void wave_lds_order()
+{
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront", "local");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront", "local");
+}
+
 // Drop the planes whose partial sum has reached `bound`, keeping the order of
 // the others; ids holds the candidates' indices, four bits each.
 __device__ __forceinline__ void drop_hyps(float (&d)[kGroupH], float (&a)[kGroupH], float (&b)[kGroupH],
@@ -1209,13 +1221,17 @@ __device__ __forceinline__ void halfstep_tile(const ViewDesc &V, const Tile &t, 
                         first += bits_below(mq);
                         units += __popcll(mq);
                     }
+                    // The unit table takes the wave's part of the list's row s:
+                    // every lane holds its draw count in e and puts it back.
                     uint32_t *slot = s_list + s * kThreads + (tid - lane);
+                    wave_lds_order();          // counts read, tap weights written
 #pragma unroll
                     for (int q = 0; q < kGroupH; ++q) {
                         if (q * G >= kGroupH) break;
                         to[q] = first + q;
                         if (l > q * G) slot[first + q] = (uint32_t)(lane | q << 6);
                     }
+                    wave_lds_order();          // units written
                     const int got = (int)slot[lane];
                     slot[lane] = e;
                     const int src = lane < units ? got & 63 : lane, part = lane < units ? got >> 6 : 0;
