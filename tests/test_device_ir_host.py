@@ -60,3 +60,17 @@ def test_lanes_exchange_units_in_order(pm_ir):
         calls = _find(lines, rf"call .*@{order[0]}\(")
         assert any(made < i < writes[0] for i in calls), f
         assert any(writes[-1] < i < read for i in calls), f
+
+
+def test_half_step_writes_no_descriptor(pm_ir):
+    """k_halfstep promises that nothing writes the view descriptors while it
+    runs (noalias, read only), so no pointer through which it could write one
+    is among its arguments: the half-step counters are an array of ints."""
+    kernels = [f for f in pm_ir if "10k_halfstep" in f]
+    assert len(kernels) >= 8
+    for f in kernels:
+        head = pm_ir[f][0]
+        assert re.search(r"noalias \S* ?%views", head), head
+        args = subprocess.run(["c++filt", f], check=True, capture_output=True, text=True).stdout.strip()
+        args = args[args.index("(") + 1:].split(", ")
+        assert "vsm::ViewDesc const*" in args and "vsm::ViewDesc*" not in args, args

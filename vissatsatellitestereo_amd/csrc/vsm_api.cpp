@@ -61,6 +61,7 @@ struct Batch {
     std::vector<ViewDesc> hviews;           // sources of the uploads, kept until the stream is past them
     std::vector<Tile> htiles;
     ViewDesc *dviews = nullptr;
+    int *dsteps = nullptr;                  // half-step counter of each view
     Tile *dtiles = nullptr;
     int ntiles = 0, maxs = 1;
     int steps_done = 0, nsteps = 0;
@@ -126,6 +127,7 @@ struct vsm_ctx {
     std::vector<ServeReq *> active;
     std::map<uint64_t, std::unique_ptr<ServeReq>> reqs;
     ViewDesc *serve_views = nullptr;
+    int *serve_steps = nullptr;            // half-step counter of each descriptor slot
     std::vector<ServeReq *> serve_slots;   // request per descriptor slot (null: free)
     Tile *serve_tiles = nullptr;           // the active requests' tiles, concatenated
     int serve_cap_tiles = 0, serve_ntiles = 0;
@@ -539,7 +541,6 @@ int prepare_view(vsm_ctx *c, const vsm_view_req &r, int pass, uint32_t view_id, 
     V.H = ref.H;
     V.n_src = r.n_src;
     V.pass = pass;
-    V.step = 0;
     V.num_steps = 2 * c->params.num_iterations;
     V.view_id = view_id;
     V.active = 1;
@@ -607,15 +608,15 @@ int ensure_c0(vsm_ctx *c, int maxs, int tw)
     return VSM_OK;
 }
 
-int record_halfstep(vsm_ctx *c, int maxs, int tw, ViewDesc *dviews, int nviews, const Tile *dtiles,
-                    int ntiles, const PMConst &pc, bool timed)
+int record_halfstep(vsm_ctx *c, int maxs, int tw, const ViewDesc *dviews, int *dsteps, int nviews,
+                    const Tile *dtiles, int ntiles, const PMConst &pc, bool timed)
 {
     {
         const int rc = ensure_c0(c, maxs, tw);
         if (rc) return rc;
     }
     if (timed) HIPCHK(c, hipEventRecord(c->ev0, c->stream));
-    HIPCHK(c, launch_halfstep(maxs, tw, dviews, nviews, dtiles, ntiles, pc, c->d_counters, c->d_work,
+    HIPCHK(c, launch_halfstep(maxs, tw, dviews, dsteps, nviews, dtiles, ntiles, pc, c->d_counters, c->d_work,
                               grid_for(c, maxs, tw), c->d_c0, c->stream));
     if (timed) {
         HIPCHK(c, hipEventRecord(c->ev1, c->stream));
@@ -688,8 +689,10 @@ void batch_release(vsm_ctx *c, Batch &b)
     for (auto &v : b.views) release_view(c, v);
     b.views.clear();
     dfree(c, b.dviews);
+    dfree(c, b.dsteps);
     dfree(c, b.dtiles);
     b.dviews = nullptr;
+    b.dsteps = nullptr;
     b.dtiles = nullptr;
 }
 
@@ -731,6 +734,7 @@ int batch_begin(vsm_ctx *c, const vsm_view_req *reqs, int n, int pass, int use_g
                     "most 16)", b.params.tile_width, b.maxs);
     }
     rc = dalloc(c, &b.dviews, n);
+    if (!rc) rc = dalloc(c, &b.dsteps, n);
     if (!rc) rc = dalloc(c, &b.dtiles, tiles.size());
     if (!rc) rc = ensure_c0(c, b.maxs, b.params.tile_width);     // before any capture
     if (rc) {
@@ -749,6 +753,7 @@ int batch_begin(vsm_ctx *c, const vsm_view_req *reqs, int n, int pass, int use_g
     BEGINCHK(hipMemcpyAsync(b.dviews, hv.data(), n * sizeof(ViewDesc), hipMemcpyHostToDevice, c->stream));
     BEGINCHK(hipMemcpyAsync(b.dtiles, tiles.data(), tiles.size() * sizeof(Tile), hipMemcpyHostToDevice,
                             c->stream));
+    BEGINCHK(launch_fill_u32(reinterpret_cast<uint32_t *>(b.dsteps), n, 0u, c->stream));
     if (pass == 0) {
         BEGINCHK(launch_init(b.dviews, b.dtiles, b.ntiles, pc, 1, b.params.tile_width, c->stream));
     } else {
@@ -800,8 +805,8 @@ int batch_step(vsm_ctx *c, Batch &b, int k)
             HIPCHK(c, hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal));
             hipError_t ce = hipSuccess;
             for (int s = 0; s < m && ce == hipSuccess; ++s) {
-                ce = launch_halfstep(b.maxs, b.params.tile_width, b.dviews, (int)b.views.size(), b.dtiles,
-                                     b.ntiles, pc, c->d_counters, c->d_work,
+                ce = launch_halfstep(b.maxs, b.params.tile_width, b.dviews, b.dsteps, (int)b.views.size(),
+                                     b.dtiles, b.ntiles, pc, c->d_counters, c->d_work,
                                      grid_for(c, b.maxs, b.params.tile_width), c->d_c0, c->stream);
             }
             const hipError_t ee = hipStreamEndCapture(c->stream, &graph);
@@ -828,8 +833,8 @@ int batch_step(vsm_ctx *c, Batch &b, int k)
         c->halfstep_launches += m;
     } else {
         for (int s = 0; s < m; ++s) {
-            const int rc = record_halfstep(c, b.maxs, b.params.tile_width, b.dviews, (int)b.views.size(),
-                                           b.dtiles, b.ntiles, pc, c->timing);
+            const int rc = record_halfstep(c, b.maxs, b.params.tile_width, b.dviews, b.dsteps,
+                                           (int)b.views.size(), b.dtiles, b.ntiles, pc, c->timing);
             if (rc) return rc;
         }
     }
@@ -1269,8 +1274,8 @@ static int debug_state(vsm_ctx *c, const vsm_view_req *req, int pass, int mode, 
     if (rc) return rc;
     ViewDesc &V = vs.desc;
     const size_t hw = (size_t)V.W * V.H;
-    V.step = 2 * iter + color;
-    V.num_steps = V.step + 1;
+    const int step = 2 * iter + color;
+    V.num_steps = step + 1;
     const int tw = c->params.tile_width;
     if (mode == 1 && !tile_width_supported(tw, V.n_src)) {
         release_view(c, vs);
@@ -1281,7 +1286,9 @@ static int debug_state(vsm_ctx *c, const vsm_view_req *req, int pass, int mode, 
     ViewDesc *dv = nullptr;
     Tile *dt = nullptr;
     uint32_t *dm = nullptr;
+    int *ds = nullptr;
     rc = dalloc(c, &dv, 1);
+    if (!rc) rc = dalloc(c, &ds, 1);
     if (!rc) rc = dalloc(c, &dt, tiles.size());
     if (!rc && mode == 2) rc = dalloc(c, &dm, hw);
     if (!rc && mode == 1) rc = ensure_c0(c, V.n_src, tw);
@@ -1296,11 +1303,12 @@ static int debug_state(vsm_ctx *c, const vsm_view_req *req, int pass, int mode, 
             if (prob) HIPCHK(c, hipMemcpyAsync(vs.prob, prob, hw * V.n_src * 4, hipMemcpyHostToDevice, c->stream));
         }
         HIPCHK(c, hipMemcpyAsync(dv, &V, sizeof V, hipMemcpyHostToDevice, c->stream));
+        HIPCHK(c, launch_fill_u32(reinterpret_cast<uint32_t *>(ds), 1, (uint32_t)step, c->stream));
         HIPCHK(c, hipMemcpyAsync(dt, tiles.data(), tiles.size() * sizeof(Tile), hipMemcpyHostToDevice, c->stream));
         const int nt = (int)tiles.size();
         if (mode == 0) HIPCHK(c, launch_init(dv, dt, nt, pc, 1, tw, c->stream));
         else if (mode == 1)
-            HIPCHK(c, launch_halfstep(V.n_src, tw, dv, 1, dt, nt, pc, c->d_counters, c->d_work,
+            HIPCHK(c, launch_halfstep(V.n_src, tw, dv, ds, 1, dt, nt, pc, c->d_counters, c->d_work,
                                       grid_for(c, V.n_src, tw), c->d_c0, c->stream));
         else HIPCHK(c, launch_filter(V.n_src, dv, dt, nt, pc, dm, c->stream));
         HIPCHK(c, hipMemcpyAsync(h.data(), vs.hyp, hw * sizeof(float4), hipMemcpyDeviceToHost, c->stream));
@@ -1314,7 +1322,7 @@ static int debug_state(vsm_ctx *c, const vsm_view_req *req, int pass, int mode, 
         }
         if (mode == 1) rc = read_counters(c, pc);
     }
-    dfree(c, dv); dfree(c, dt); dfree(c, dm);
+    dfree(c, dv); dfree(c, ds); dfree(c, dt); dfree(c, dm);
     release_view(c, vs);
     return rc;
 }
@@ -1841,8 +1849,9 @@ static int serve_start(vsm_ctx *c, ServeReq &r)
     if (!rc) {
         const PMConst pc = make_const(c->params);
         ViewDesc *dv = c->serve_views + r.slot;
-        r.vs.desc.step = 0;
         hipError_t e = hipMemcpyAsync(dv, &r.vs.desc, sizeof(ViewDesc), hipMemcpyHostToDevice, c->stream);
+        if (e == hipSuccess)
+            e = launch_fill_u32(reinterpret_cast<uint32_t *>(c->serve_steps + r.slot), 1, 0u, c->stream);
         if (e == hipSuccess && r.pass == 1)     // start from the photometric depth and normals
             e = launch_load_hyp(dv, 0, (int)hw, img.depth[0], img.normal[0], pc.cos_max_normal, c->stream);
         if (e == hipSuccess)
@@ -1924,8 +1933,6 @@ static int serve_finish(vsm_ctx *c, ServeReq &r, ViewDesc *dv)
     ImageRec &img = c->images.at(r.ref);
     const size_t hw = (size_t)r.vs.desc.W * r.vs.desc.H;
     const PMConst pc = make_const(c->params);
-    r.vs.desc.step = r.vs.desc.num_steps;
-    HIPCHK(c, hipMemcpyAsync(dv, &r.vs.desc, sizeof(ViewDesc), hipMemcpyHostToDevice, c->stream));
     if (r.filter && r.tile_w == kTileW && r.dtiles) {
         // the request's own half-step tiles have the filter's shape
         HIPCHK(c, launch_filter(r.vs.desc.n_src, c->serve_views, r.dtiles, r.ntiles, pc, r.out_mask,
@@ -1974,6 +1981,7 @@ static int serve_submit(vsm_ctx *c, const vsm_view_req *req, int pass, int filte
     // resident serving scratch is allocated before any admission decision
     int rc = VSM_OK;
     if (!c->serve_views && (rc = dalloc(c, &c->serve_views, kServeMaxViews))) return rc;
+    if (!c->serve_steps && (rc = dalloc(c, &c->serve_steps, kServeMaxViews))) return rc;
     c->serve_slots.resize(kServeMaxViews, nullptr);
     if (!tile_width_supported(c->params.tile_width, req->n_src))
         return fail(c, VSM_EINVAL, "tile_width %d is not available for %d sources", c->params.tile_width,
@@ -2047,8 +2055,8 @@ int vsm_serve_step(vsm_ctx *c, int32_t *n_active, int32_t *n_queued)
             c->serve_dirty = false;
         }
         const PMConst pc = make_const(c->params);
-        if ((rc = record_halfstep(c, maxs, c->params.tile_width, c->serve_views, nslots, c->serve_tiles,
-                                  c->serve_ntiles, pc, c->timing)))
+        if ((rc = record_halfstep(c, maxs, c->params.tile_width, c->serve_views, c->serve_steps, nslots,
+                                  c->serve_tiles, c->serve_ntiles, pc, c->timing)))
             return rc;
         HIPCHK(c, hipStreamSynchronize(c->stream));
         // Every active request has advanced one half-step.  The finished ones

@@ -41,9 +41,9 @@ struct PMConst {
 // One reference view and its sources (device memory; read through scalar loads).
 struct ViewDesc {
     int W, H, n_src, pass;
-    int step, num_steps;            // half-step counter: iter = step >> 1, colour = step & 1
+    int num_steps;                  // half-steps of the pass
     uint32_t view_id;
-    int active;
+    int active, pad;
     const uint8_t *ref;             // W*H gray, row-major
     float4 *hyp;                    // (d, n0, n1, n2) per pixel
     float *cost;                    // per pixel

@@ -8,9 +8,10 @@ namespace vsm {
 // Half-step kernel for up to maxs sources on tiles of tw x (512 / tw)
 // pixels: 16 or 32 wide, and 64 for at most 16 sources.
 bool tile_width_supported(int tw, int maxs);
-// work: kXcd + 1 zeroed words, left zero; the half-step counters of
-// views[0 .. nadv-1] advance when the half-step is done.
-hipError_t launch_halfstep(int maxs, int tw, ViewDesc *views, int nadv, const Tile *tiles, int ntiles,
+// work: kXcd + 1 zeroed words, left zero; steps: the half-step counters of
+// views[0 .. nviews-1], which advance when the half-step is done.
+hipError_t launch_halfstep(int maxs, int tw, const ViewDesc *views, int *steps, int nviews,
+                           const Tile *tiles, int ntiles,
                            const PMConst &c, Counters *counters, unsigned int *work, int grid,
                            float *c0_scratch, hipStream_t st);
 // Resident workgroups of the persistent half-step kernel on this device.

@@ -888,16 +888,17 @@ __device__ __forceinline__ void tile_prologue(const ViewDesc &V, const PMConst &
                      s_src[threadIdx.x]);
 }
 
-// One red-black half-step on one tile (all 256 threads of the workgroup
-// call it; it contains one barrier).
+// One red-black half-step (number `step`: iteration step >> 1, colour step & 1)
+// on one tile (all 256 threads of the workgroup call it; it contains one
+// barrier).
 template <int MAXS, int TW>
-__device__ __forceinline__ void halfstep_tile(const ViewDesc &V, const Tile &t, const PMConst &c,
+__device__ __forceinline__ void halfstep_tile(const ViewDesc &V, const Tile &t, int step, const PMConst &c,
                                               float *s_ref, SrcLds *s_src, float *s_c0,
                                               uint32_t *s_list, float *s_w, unsigned int &my_ncc,
                                               unsigned int &my_geo)
 {
     using T = TileShape<TW>;
-    const int iter = V.step >> 1, color = V.step & 1, pass = V.pass;
+    const int iter = step >> 1, color = step & 1, pass = V.pass;
     const int W = V.W, H = V.H, S = V.n_src;
     const int tid = threadIdx.x;
     tile_prologue<MAXS, TW>(V, c, t, s_ref, s_src);
@@ -1310,15 +1311,16 @@ __device__ __forceinline__ void halfstep_tile(const ViewDesc &V, const Tile &t, 
 // work[0 .. kXcd-1] are the per-XCD cursors, work[kXcd] counts the workgroups
 // that are done: all zero before the first launch, and left zero by the last
 // workgroup to finish, which also advances the half-step counters of the views
-// (adv[0 .. nadv-1]).  Nothing else runs between two half-steps: a fill and an
-// advance kernel of 5 us each used to (photo solve of two 256 x 256 views, 10
-// half-steps: 1802 -> 1753 us).
+// (steps[0 .. nviews-1]; an array of their own, since the descriptors are read
+// as memory that no one writes).  Nothing else runs between two half-steps: a
+// fill and an advance kernel of 5 us each used to (photo solve of two 256 x 256
+// views, 10 half-steps: 1802 -> 1753 us).
 template <int MAXS, int TW>
 __global__ __launch_bounds__(kThreads, 2) void k_halfstep(const ViewDesc *__restrict__ views,
                                                        const Tile *__restrict__ tiles, int ntiles,
                                                        PMConst c, Counters *counters,
-                                                       unsigned int *work, float *c0g, ViewDesc *adv,
-                                                       int nadv)
+                                                       unsigned int *work, float *c0g, int *steps,
+                                                       int nviews)
 {
     __shared__ float s_ref[TileShape<TW>::LH * TileShape<TW>::LW];
     __shared__ SrcLds s_src[MAXS];
@@ -1348,8 +1350,9 @@ __global__ __launch_bounds__(kThreads, 2) void k_halfstep(const ViewDesc *__rest
             if (ti < 0) break;
             const Tile t = tiles[ti];
             const ViewDesc &V = views[t.view];
-            if (!V.active || V.step >= V.num_steps) continue;     // uniform per workgroup
-            halfstep_tile<MAXS, TW>(V, t, c, s_ref, s_src,
+            const int step = __builtin_amdgcn_readfirstlane(steps[t.view]);
+            if (!V.active || step >= V.num_steps) continue;       // uniform per workgroup
+            halfstep_tile<MAXS, TW>(V, t, step, c, s_ref, s_src,
                                 MAXS > 16 ? c0g + (size_t)blockIdx.x * (MAXS * kThreads) : s_c0,
                                 s_list, s_w, my_ncc, my_geo);
         }
@@ -1369,8 +1372,8 @@ __global__ __launch_bounds__(kThreads, 2) void k_halfstep(const ViewDesc *__rest
     __syncthreads();
     if (s_tile) {
         if (tid <= kXcd) work[tid] = 0u;
-        for (int v = tid; v < nadv; v += kThreads)
-            if (adv[v].active && adv[v].step < adv[v].num_steps) adv[v].step += 1;
+        for (int v = tid; v < nviews; v += kThreads)
+            if (views[v].active && steps[v] < views[v].num_steps) steps[v] += 1;
     }
 }
 
@@ -1748,7 +1751,7 @@ __global__ void k_fill_u64(unsigned long long *p, int n, unsigned long long v)
 // The kernel instantiation for (sources, tile width); null for an
 // unsupported width.
 typedef void (*halfstep_fn)(const ViewDesc *, const Tile *, int, PMConst, Counters *, unsigned int *,
-                            float *, ViewDesc *, int);
+                            float *, int *, int);
 
 template <int MAXS>
 static halfstep_fn halfstep_for_width(int tw)
@@ -1774,7 +1777,8 @@ static halfstep_fn halfstep_kernel(int maxs, int tw)
 
 bool tile_width_supported(int tw, int maxs) { return tw == 16 || tw == 32 || (tw == 64 && maxs <= 16); }
 
-hipError_t launch_halfstep(int maxs, int tw, ViewDesc *views, int nadv, const Tile *tiles, int ntiles,
+hipError_t launch_halfstep(int maxs, int tw, const ViewDesc *views, int *steps, int nviews,
+                           const Tile *tiles, int ntiles,
                            const PMConst &c, Counters *counters, unsigned int *work, int grid,
                            float *c0_scratch, hipStream_t st)
 {
@@ -1784,7 +1788,7 @@ hipError_t launch_halfstep(int maxs, int tw, ViewDesc *views, int nadv, const Ti
     // more than 16 sources: c0_scratch holds grid x 32 x kThreads floats
     if (maxs > 16 && !c0_scratch) return hipErrorInvalidValue;
     grid = max(kXcd, min(grid, ((ntiles + kXcd - 1) / kXcd) * kXcd));
-    fn<<<grid, kThreads, 0, st>>>(views, tiles, ntiles, c, counters, work, c0_scratch, views, nadv);
+    fn<<<grid, kThreads, 0, st>>>(views, tiles, ntiles, c, counters, work, c0_scratch, steps, nviews);
     return hipGetLastError();
 }
 
