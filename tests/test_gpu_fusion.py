@@ -67,6 +67,18 @@ def test_median_blur_bit_exact(ctx):
         assert _same(ctx.median_blur3(a), fo.median_blur3(a)), shape
 
 
+def test_median_blur_of_a_tall_raster_is_whole(ctx):
+    """A raster of one column and more rows than one launch holds threads for:
+    every row is the median of itself and its two neighbours (the border row
+    repeated)."""
+    n = (1 << 28) + 5000
+    a = (np.arange(n, dtype=np.int32) % 1009).astype(np.float32)
+    out = ctx.median_blur3(a[:, None])[:, 0]
+    above, below = np.concatenate([a[:1], a[:-1]]), np.concatenate([a[1:], a[-1:]])
+    lo, hi = np.minimum(above, below), np.maximum(above, below)
+    assert np.array_equal(out, np.minimum(np.maximum(a, lo), hi))
+
+
 def test_fuse_dsm_bit_exact(ctx, tiny):
     """Per-view and fused DSMs of noisy ground-truth depth maps (with holes)."""
     names = tiny["names"]

@@ -21,7 +21,7 @@
 #include "vsm_geo.h"
 #include "vsm_kernels.h"
 
-
+#include <algorithm>
 #include <mutex>
 #include <vector>
 
@@ -415,18 +415,20 @@ __device__ __forceinline__ float median_of_window(const float (&x)[9])
 constexpr int kMedRows = 4;
 
 __global__ __launch_bounds__(256) void k_median3(const float *__restrict__ in, int e_size, int n_size,
-                                                 float *__restrict__ out)
+                                                 unsigned int first, float *__restrict__ out)
 {
-    const unsigned int across = (e_size + 63) / 64;      // one-dimensional grid: any number of rows
-    const int c = (int)(blockIdx.x % across) * 64 + (threadIdx.x & 63);
-    const int r0 = ((int)(blockIdx.x / across) * 4 + (threadIdx.x >> 6)) * kMedRows;
+    // one-dimensional grid from block `first` of the raster on: any number of rows
+    const unsigned int across = (e_size + 63) / 64, block = first + blockIdx.x;
+    const int c = (int)(block % across) * 64 + (threadIdx.x & 63);
+    const int r0 = ((int)(block / across) * 4 + (threadIdx.x >> 6)) * kMedRows;
     if (c >= e_size || r0 >= n_size) return;
     float w[kMedRows + 2][3], m[kMedRows];
 #pragma unroll
     for (int r = 0; r < kMedRows + 2; ++r)
 #pragma unroll
         for (int dc = -1; dc <= 1; ++dc) {
-            const int rr = min(max(r0 - 1 + r, 0), n_size - 1), cc = min(max(c + dc, 0), e_size - 1);
+            const int rr = max((int)min((unsigned int)r0 + r, (unsigned int)n_size) - 1, 0);   // row r0 - 1 + r
+            const int cc = min(max(c + dc, 0), e_size - 1);
             w[r][dc + 1] = in[(size_t)rr * e_size + cc];
         }
     const uint32_t nan = column_medians<kMedRows>(w, m);
@@ -725,9 +727,17 @@ hipError_t launch_view_dsm(const unsigned long long *keys, unsigned long long *c
 
 hipError_t launch_median3(const float *in, int e_size, int n_size, float *out, hipStream_t st)
 {
-    const unsigned int grid = nblk(e_size, 64) * nblk(n_size, 4 * kMedRows);
-    k_median3<<<grid, 256, 0, st>>>(in, e_size, n_size, out);
-    return hipGetLastError();
+    // A launch holds fewer than 2^32 threads.  Blocks are 64 columns wide, so a
+    // narrow raster of many rows has more threads than cells (2^28 rows of up to
+    // 8 cells reach the limit) and takes several launches.
+    constexpr unsigned int kMaxBlocks = 1u << 23;
+    const unsigned int blocks = nblk(e_size, 64) * nblk(n_size, 4 * kMedRows);
+    for (unsigned int first = 0; first < blocks; first += kMaxBlocks) {
+        k_median3<<<std::min(kMaxBlocks, blocks - first), 256, 0, st>>>(in, e_size, n_size, first, out);
+        const hipError_t e = hipGetLastError();
+        if (e != hipSuccess) return e;
+    }
+    return hipSuccess;
 }
 
 hipError_t launch_fuse_stack(const float *stack, int nviews, long long ncell, int min_measurements,
