@@ -135,7 +135,7 @@ struct vsm_ctx {
     // staged batched solves
     std::map<int, std::unique_ptr<Batch>> batches;
     int next_batch = 1;
-    CopyOut copier;                        // results to caller-owned host memory
+    CopyRing copier;                       // results to caller-owned host memory
 };
 
 namespace {
@@ -160,28 +160,6 @@ int fail(vsm_ctx *c, int code, const char *fmt, ...)
             return fail((ctx), VSM_EDEVICE, "%s failed: %s (%s:%d)", #expr, hipGetErrorString(e_), \
                         __FILE__, __LINE__);                                                    \
     } while (0)
-
-// Results to host memory: copy_out queues a copy behind the context's stream,
-// copies_done waits for the stream and for the data to be in place.  An entry
-// point that calls copy_out holds a CopyScope, so that no copy is under way
-// into the caller's memory when it returns early.
-hipError_t copy_out(vsm_ctx *c, void *dst, const void *src, size_t n)
-{
-    return c->copier.copy(dst, src, n, c->device, c->stream);
-}
-
-hipError_t copies_done(vsm_ctx *c)
-{
-    const hipError_t e = hipStreamSynchronize(c->stream);
-    const hipError_t w = c->copier.wait();
-    return e != hipSuccess ? e : w;
-}
-
-struct CopyScope {
-    explicit CopyScope(vsm_ctx *ctx) : c(ctx) {}
-    ~CopyScope() { (void)c->copier.wait(); }
-    vsm_ctx *c;
-};
 
 // Device memory: blocks freed by the library go to a per-context cache and
 // are reused by later allocations of up to the same size (all work runs in
@@ -641,9 +619,10 @@ int read_counters(vsm_ctx *c, const PMConst &pc)
     return VSM_OK;
 }
 
-// dv: the view's descriptor on the device.
+// dv: the view's descriptor on the device.  The outputs are in place when the
+// caller has finished `copies`.
 int finalize_outputs(vsm_ctx *c, int pass, int ref_id, vsm_view_out *out, const uint32_t *d_mask,
-                     const ViewDesc *dv)
+                     const ViewDesc *dv, CopyCall &copies)
 {
     ImageRec &ref = c->images[ref_id];
     const size_t hw = (size_t)ref.W * ref.H;
@@ -659,13 +638,13 @@ int finalize_outputs(vsm_ctx *c, int pass, int ref_id, vsm_view_out *out, const 
                               c->stream));
     if (pass == 0) ++ref.depth_ver;
     if (out && out->depth)
-        HIPCHK(c, copy_out(c, out->depth, tmp, hw * 4));
+        HIPCHK(c, copies.copy(out->depth, tmp, hw * 4));
     if (out && out->normal)
-        HIPCHK(c, copy_out(c, out->normal, ref.normal[pass], hw * 12));
+        HIPCHK(c, copies.copy(out->normal, ref.normal[pass], hw * 12));
     if (out && out->cost)
-        HIPCHK(c, copy_out(c, out->cost, tmp + hw, hw * 4));
+        HIPCHK(c, copies.copy(out->cost, tmp + hw, hw * 4));
     if (out && out->consistency) {
-        if (d_mask) HIPCHK(c, copy_out(c, out->consistency, d_mask, hw * 4));
+        if (d_mask) HIPCHK(c, copies.copy(out->consistency, d_mask, hw * 4));
         else memset(out->consistency, 0, hw * 4);
     }
     // tmp goes back to the cache; the copies above are ordered before any
@@ -847,7 +826,7 @@ int batch_finish(vsm_ctx *c, Batch &b, vsm_view_out *outs)
 {
     const int n = (int)b.views.size();
     const PMConst pc = make_const(b.params);
-    CopyScope scope(c);
+    CopyCall copies(c->copier, c->device, c->stream);
     uint32_t *d_masks = nullptr;
     std::vector<size_t> mask_off(n, 0);
     int rc = VSM_OK;
@@ -880,8 +859,8 @@ int batch_finish(vsm_ctx *c, Batch &b, vsm_view_out *outs)
     }
     for (int v = 0; v < n && !rc; ++v)
         rc = finalize_outputs(c, b.pass, b.ref_ids[v], outs ? &outs[v] : nullptr,
-                              d_masks ? d_masks + mask_off[v] : nullptr, b.dviews + v);
-    const hipError_t se = copies_done(c);
+                              d_masks ? d_masks + mask_off[v] : nullptr, b.dviews + v, copies);
+    const hipError_t se = copies.finish();
     if (!rc && se != hipSuccess)
         rc = fail(c, VSM_EDEVICE, "hipStreamSynchronize failed: %s", hipGetErrorString(se));
     dfree(c, d_masks);
@@ -1107,9 +1086,9 @@ int vsm_get_depth_map(vsm_ctx *c, int32_t id, int32_t kind, float *depth, int32_
     if (w != r.W || h != r.H) return fail(c, VSM_EINVAL, "buffer %dx%d != image %dx%d", w, h, r.W, r.H);
     if (!r.depth[kind]) return fail(c, VSM_ENOENT, "image %d has no depth map of kind %d", id, kind);
     HIPCHK(c, hipSetDevice(c->device));
-    CopyScope scope(c);
-    HIPCHK(c, copy_out(c, depth, r.depth[kind], (size_t)w * h * 4));
-    HIPCHK(c, copies_done(c));
+    CopyCall copies(c->copier, c->device, c->stream);
+    HIPCHK(c, copies.copy(depth, r.depth[kind], (size_t)w * h * 4));
+    HIPCHK(c, copies.finish());
     return VSM_OK;
 }
 
@@ -1425,10 +1404,10 @@ int vsm_fuse_dsm(vsm_ctx *c, const vsm_dsm_grid *grid, const int32_t *ids, int32
     }
     c->fuse_launches += 1;
     c->fuse_pixels += pixels;
-    CopyScope scope(c);
-    HIPCHK(c, copy_out(c, dsm_out, fused, ncell * 4));
-    if (per_view_out) HIPCHK(c, copy_out(c, per_view_out, stack, (size_t)ncell * 4 * n));
-    HIPCHK(c, copies_done(c));
+    CopyCall copies(c->copier, c->device, c->stream);
+    HIPCHK(c, copies.copy(dsm_out, fused, ncell * 4));
+    if (per_view_out) HIPCHK(c, copies.copy(per_view_out, stack, (size_t)ncell * 4 * n));
+    HIPCHK(c, copies.finish());
     dfree(c, cells); dfree(c, stack); dfree(c, tmp); dfree(c, fused); dfree(c, mats);
     return VSM_OK;
 }
@@ -1507,7 +1486,7 @@ int vsm_fuse_points(vsm_ctx *c, const int32_t *ids, int32_t n, int32_t depth_kin
             return fail(c, VSM_EDEVICE, "%s failed: %s", #expr, hipGetErrorString(e_));        \
         }                                                                                       \
     } while (0)
-    CopyScope scope(c);
+    CopyCall copies(c->copier, c->device, c->stream);
     F3CHK(hipMemcpyAsync(dviews, hv.data(), n * sizeof(Fuse3dView), hipMemcpyHostToDevice, c->stream));
     int64_t total = 0;
     for (int v = 0; v < n; ++v) {
@@ -1518,13 +1497,13 @@ int vsm_fuse_points(vsm_ctx *c, const int32_t *ids, int32_t n, int32_t depth_kin
         F3CHK(hipStreamSynchronize(c->stream));
         const int64_t put = std::min<int64_t>(room, ns);
         if (put > 0) {
-            F3CHK(copy_out(c, xyz + 3 * total, f.xyz, put * 24));
-            if (normal) F3CHK(copy_out(c, normal + 3 * total, f.normal, put * 12));
-            if (grey) F3CHK(copy_out(c, grey + total, f.gray, put));
+            F3CHK(copies.copy(xyz + 3 * total, f.xyz, put * 24));
+            if (normal) F3CHK(copies.copy(normal + 3 * total, f.normal, put * 12));
+            if (grey) F3CHK(copies.copy(grey + total, f.gray, put));
         }
         total += ns;
     }
-    F3CHK(copies_done(c));
+    F3CHK(copies.finish());
 #undef F3CHK
     cleanup();
     *count = total;
@@ -1551,9 +1530,9 @@ int vsm_proj_to_grid(vsm_ctx *c, const double *points, int64_t n, const vsm_dsm_
     HIPCHK(c, launch_fill_u64n(cells, ncell, 0ull, c->stream));
     HIPCHK(c, launch_rasterize_points(pts, n, g, cells, c->stream));
     HIPCHK(c, launch_decode_fill_f64(cells, g.e_size, g.n_size, out, c->stream));
-    CopyScope scope(c);
-    HIPCHK(c, copy_out(c, dsm_out, out, ncell * 8));
-    HIPCHK(c, copies_done(c));
+    CopyCall copies(c->copier, c->device, c->stream);
+    HIPCHK(c, copies.copy(dsm_out, out, ncell * 8));
+    HIPCHK(c, copies.finish());
     dfree(c, cells); dfree(c, out); dfree(c, pts);
     return VSM_OK;
 }
@@ -1658,9 +1637,9 @@ int vsm_enu_to_utm(vsm_ctx *c, const double *enu, int64_t n, double *out)
     if (rc) return rc;
     HIPCHK(c, hipMemcpyAsync(buf, enu, 24 * (size_t)n, hipMemcpyHostToDevice, c->stream));
     HIPCHK(c, launch_enu_to_utm(buf, n, c->geo, buf + 3 * (size_t)n, c->stream));
-    CopyScope scope(c);
-    HIPCHK(c, copy_out(c, out, buf + 3 * (size_t)n, 24 * (size_t)n));
-    HIPCHK(c, copies_done(c));
+    CopyCall copies(c->copier, c->device, c->stream);
+    HIPCHK(c, copies.copy(out, buf + 3 * (size_t)n, 24 * (size_t)n));
+    HIPCHK(c, copies.finish());
     dfree(c, buf);
     return VSM_OK;
 }
@@ -1677,9 +1656,9 @@ int vsm_median_blur3(vsm_ctx *c, const float *in, int32_t e_size, int32_t n_size
     if (rc) return rc;
     HIPCHK(c, hipMemcpyAsync(buf, in, nc * 4, hipMemcpyHostToDevice, c->stream));
     HIPCHK(c, launch_median3(buf, e_size, n_size, buf + nc, c->stream));
-    CopyScope scope(c);
-    HIPCHK(c, copy_out(c, out, buf + nc, nc * 4));
-    HIPCHK(c, copies_done(c));
+    CopyCall copies(c->copier, c->device, c->stream);
+    HIPCHK(c, copies.copy(out, buf + nc, nc * 4));
+    HIPCHK(c, copies.finish());
     dfree(c, buf);
     return VSM_OK;
 }
@@ -2117,12 +2096,12 @@ int vsm_poll(vsm_ctx *c, uint64_t ticket, vsm_view_out *out, int32_t *done)
         return e;
     }
     const size_t hw = (size_t)r.vs.desc.W * r.vs.desc.H;
-    CopyScope scope(c);
-    if (out && out->depth) HIPCHK(c, copy_out(c, out->depth, r.out_depth, hw * 4));
-    if (out && out->normal) HIPCHK(c, copy_out(c, out->normal, r.out_normal, hw * 12));
-    if (out && out->cost) HIPCHK(c, copy_out(c, out->cost, r.out_cost, hw * 4));
-    if (out && out->consistency) HIPCHK(c, copy_out(c, out->consistency, r.out_mask, hw * 4));
-    HIPCHK(c, copies_done(c));
+    CopyCall copies(c->copier, c->device, c->stream);
+    if (out && out->depth) HIPCHK(c, copies.copy(out->depth, r.out_depth, hw * 4));
+    if (out && out->normal) HIPCHK(c, copies.copy(out->normal, r.out_normal, hw * 12));
+    if (out && out->cost) HIPCHK(c, copies.copy(out->cost, r.out_cost, hw * 4));
+    if (out && out->consistency) HIPCHK(c, copies.copy(out->consistency, r.out_mask, hw * 4));
+    HIPCHK(c, copies.finish());
     dfree(c, r.out_depth);
     c->reqs.erase(it);
     return VSM_OK;
