@@ -20,6 +20,8 @@ HIP = r"""
 enum hipError_t { hipSuccess = 0, hipErrorUnknown = 999 };
 enum hipMemcpyKind { hipMemcpyDeviceToHost = 2 };
 enum { hipEventDisableTiming = 2 };
+enum hipMemoryType { hipMemoryTypeUnregistered = 0, hipMemoryTypeHost = 1 };
+struct hipPointerAttribute_t { hipMemoryType type; };
 struct Op { void *dst; const void *src; size_t n; };
 struct Stream { std::mutex mu; std::vector<Op> ops; size_t done = 0; };
 struct Event { Stream *st = nullptr; size_t at = 0; bool bad = false; };
@@ -27,7 +29,6 @@ typedef Stream *hipStream_t;
 typedef Event *hipEvent_t;
 inline const char *marked = nullptr;               // reads of [marked, marked + marked_n) fail
 inline size_t marked_n = 0;
-inline int direct_to = 0;                          // copies into memory that hipHostMalloc did not make
 inline std::vector<std::pair<char *, size_t>> pinned;
 inline bool is_marked(const void *p) { return marked && (const char *)p >= marked && (const char *)p < marked + marked_n; }
 inline bool is_pinned(const void *p)
@@ -44,7 +45,6 @@ inline hipError_t run_to(Stream &s, size_t at)
 inline hipError_t hipMemcpyAsync(void *d, const void *s, size_t n, hipMemcpyKind, hipStream_t st)
 {
     std::lock_guard<std::mutex> lk(st->mu);
-    if (!is_pinned(d)) ++direct_to;
     st->ops.push_back(Op{d, s, n});
     return hipSuccess;
 }
@@ -71,6 +71,11 @@ inline hipError_t hipHostMalloc(void **p, size_t n, unsigned)
 {
     *p = malloc(n);
     pinned.emplace_back((char *)*p, n);
+    return hipSuccess;
+}
+inline hipError_t hipPointerGetAttributes(hipPointerAttribute_t *a, const void *p)
+{
+    a->type = is_pinned(p) ? hipMemoryTypeHost : hipMemoryTypeUnregistered;
     return hipSuccess;
 }
 inline hipError_t hipHostFree(void *p) { free(p); return hipSuccess; }
@@ -130,6 +135,23 @@ static int early()
     return 0;
 }
 
+// Pinned memory of the caller takes the data straight, in one copy.
+static int straight()
+{
+    CopyRing ring;
+    Stream st;
+    const size_t n = 3u << 20;
+    auto a = numbers(n, 4);
+    void *p = nullptr;
+    CHECK(hipHostMalloc(&p, n + 64, 0) == hipSuccess);
+    CopyCall call(ring, 0, &st);
+    CHECK(call.copy((char *)p + 64, a.data(), n) == hipSuccess);
+    CHECK(st.ops.size() == 1 && st.ops[0].dst == (char *)p + 64);
+    CHECK(call.finish() == hipSuccess);
+    CHECK(!memcmp((char *)p + 64, a.data(), n));
+    return 0;
+}
+
 // Calls of two threads, longer than the ring and in pieces of every kind.
 static int threads()
 {
@@ -151,7 +173,10 @@ static int threads()
     return 0;
 }
 
-int main() { return errors() || early() || threads(); }
+int main(int argc, char **argv)
+{
+    return argc > 1 && !strcmp(argv[1], "straight") ? straight() : errors() || early() || threads();
+}
 """
 
 
@@ -173,4 +198,10 @@ def test_copies_of_a_call_are_its_own(program):
     """Errors stay with the call whose copy met them, a call that ends early
     has waited for its copies, and calls of two threads share the ring."""
     r = subprocess.run([program], capture_output=True, text=True, timeout=60)
+    assert r.returncode == 0, r.stdout
+
+
+def test_pinned_memory_is_written_straight(program):
+    """A destination that the device reaches itself does not go through the ring."""
+    r = subprocess.run([program, "straight"], capture_output=True, text=True, timeout=60)
     assert r.returncode == 0, r.stdout

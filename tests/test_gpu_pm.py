@@ -542,6 +542,26 @@ def test_copies_to_host_are_whole(w, h):
     ctx.close()
 
 
+@pytest.mark.parametrize("w,h", [(511, 512), (513, 512), (3001, 2999)])
+def test_copies_to_pinned_memory_are_whole(w, h):
+    """Pinned destinations, which the device writes itself, from an odd offset
+    on and beside pageable ones."""
+    import torch
+    from vissatsatellitestereo_amd._lib import fptr
+    ctx = _ctx()
+    m = np.random.default_rng(w).random((h, w), dtype=np.float32)
+    ctx.register_geometry(1, w, h, np.eye(4))
+    ctx.set_depth_map(1, m, kind=0)
+    pinned = torch.full((h * w + 8,), -1.0, pin_memory=True).numpy()
+    for _ in range(2):
+        ctx._check(ctx.lib.vsm_get_depth_map(ctx.h, 1, 0, fptr(pinned[3:]), w, h))
+        assert np.array_equal(pinned[3:3 + h * w].reshape(h, w), m)
+        assert (pinned[:3] == -1).all() and (pinned[3 + h * w:] == -1).all()
+        assert np.array_equal(ctx.get_depth_map(1, kind=0), m)
+        pinned[3:-5] = 0
+    ctx.close()
+
+
 def test_api_rejects_bad_input_and_stays_usable(tiny):
     """Invalid parameters and requests raise (nothing reaches a kernel) and
     leave the context as it was: a valid solve afterwards matches a fresh
