@@ -888,21 +888,25 @@ __device__ __forceinline__ void tile_prologue(const ViewDesc &V, const PMConst &
                      s_src[threadIdx.x]);
 }
 
-// One red-black half-step (number `step`: iteration step >> 1, colour step & 1)
-// on one tile (all 256 threads of the workgroup call it; it contains one
-// barrier).
+// One red-black half-step (number *step_at: iteration step >> 1, colour
+// step & 1) on one tile (all 256 threads of the workgroup call it; it contains
+// one barrier).
 template <int MAXS, int TW>
-__device__ __forceinline__ void halfstep_tile(const ViewDesc &V, const Tile &t, int step, const PMConst &c,
+__device__ __forceinline__ void halfstep_tile(const ViewDesc &V, const Tile &t, const int *step_at,
+                                              const PMConst &c,
                                               float *s_ref, SrcLds *s_src, float *s_c0,
                                               uint32_t *s_list, float *s_w, unsigned int &my_ncc,
                                               unsigned int &my_geo)
 {
     using T = TileShape<TW>;
-    const int iter = step >> 1, color = step & 1, pass = V.pass;
-    const int W = V.W, H = V.H, S = V.n_src;
+    const int W = V.W, H = V.H, S = V.n_src, pass = V.pass;
     const int tid = threadIdx.x;
+    const int step_loaded = *step_at;           // on its way while the tile is staged
     tile_prologue<MAXS, TW>(V, c, t, s_ref, s_src);
     __syncthreads();
+    const int step = __builtin_amdgcn_readfirstlane(step_loaded);
+    if (step >= V.num_steps) return;            // uniform per workgroup
+    const int iter = step >> 1, color = step & 1;
 
     constexpr int kHalf = TW / 2;               // active pixels per tile row
     const int ty = tid / kHalf;
@@ -1350,9 +1354,8 @@ __global__ __launch_bounds__(kThreads, 2) void k_halfstep(const ViewDesc *__rest
             if (ti < 0) break;
             const Tile t = tiles[ti];
             const ViewDesc &V = views[t.view];
-            const int step = __builtin_amdgcn_readfirstlane(steps[t.view]);
-            if (!V.active || step >= V.num_steps) continue;       // uniform per workgroup
-            halfstep_tile<MAXS, TW>(V, t, step, c, s_ref, s_src,
+            if (!V.active) continue;                              // uniform per workgroup
+            halfstep_tile<MAXS, TW>(V, t, steps + t.view, c, s_ref, s_src,
                                 MAXS > 16 ? c0g + (size_t)blockIdx.x * (MAXS * kThreads) : s_c0,
                                 s_list, s_w, my_ncc, my_geo);
         }
