@@ -212,6 +212,48 @@ def test_lockstep_candidates_leave_early(many, ragged, name, n_src, pass_, extra
         assert r["frac_cost_err"] <= 1e-3, r
 
 
+@pytest.mark.parametrize("name,n_src,extra", [
+    ("tiny", 1, {}),                                       # nothing leaves after the only source
+    ("tiny", 2, dict(draw_group=1, tile_width=16)),
+    ("tiny", 3, dict(window_radius=3, window_step=1)),     # 49 taps, no table of weights
+    ("tiny", 3, dict(window_step=1, draw_group=1, tile_width=64)),
+    ("ragged", 3, dict(num_samples=5)),                    # partial waves
+    ("many", 9, dict(draw_group=1, tile_width=64)),
+    ("many", 16, dict(num_samples=4)),                     # most lanes idle at most sources
+    ("many", 18, dict(tile_width=16)),
+    ("many", 18, dict(draw_group=1, num_samples=6)),
+])
+def test_candidates_that_leave_change_nothing(tiny, ragged, many, name, n_src, extra):
+    """Half-steps with a geometric term too small to change any cost, of either
+    sign: below zero every candidate is evaluated on every drawn source by its
+    own lane; above, candidates leave early and idle lanes take planes over.
+    The same hypotheses, costs and probabilities bit for bit, with fewer
+    evaluations wherever a candidate can leave."""
+    site = dict(tiny=tiny, ragged=ragged, many=many)[name]
+    p = _params(**{**dict(window_radius=5, window_step=2), **extra})
+    ctx, ref, srcs = _setup(site, p, 0, n_src)
+    rid, sids, dr = _id(site, ref), [_id(site, s) for s in srcs], site["dr"][ref]
+    for s, d in _src_depths(site, srcs).items():
+        ctx.set_depth_map(_id(site, s), d, kind=0)
+    st = ctx.debug_init(rid, sids, dr, 1)
+    for k in range(6):
+        got, evals = [], []
+        for reg in (-1e-30, 1e-30):
+            ctx.set_params(geom_consistency_regularizer=reg)
+            ctx.reset_stats()
+            got.append(ctx.debug_halfstep(rid, sids, dr, st, 1, k // 2, k % 2))
+            evals.append(ctx.stats()["ncc_evals"])
+        for key in ("depth", "normal", "cost", "prob"):
+            assert np.array_equal(got[0][key], got[1][key]), (k, key)
+        if n_src == 1:
+            assert evals[1] == evals[0], (k, evals)
+        elif k >= 2:                             # each colour's planes have been searched once
+            assert evals[1] < 0.95 * evals[0], (k, evals)
+        print(k, evals, evals[1] / evals[0])
+        st = got[1]
+    ctx.close()
+
+
 def test_lds_staged_costs_equal_cached(tiny):
     """The measurement kernel that reads window taps from LDS-staged boxes of
     the sources returns the same costs as its cached-gather twin and as
