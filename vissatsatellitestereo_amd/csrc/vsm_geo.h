@@ -7,8 +7,9 @@
 //     (lib/latlonalt_enu_converter.py:43-46);
 //   latlon_to_eastnorh (lib/latlon_utm_converter.py:39-52): pyproj 'utm' on
 //     WGS84 in the zone / hemisphere of the AOI.
-// Method (own arithmetic, only IEEE +, -, *, / and sqrt, so the compiled code
-// with -ffp-contract=off gives the same bits on the CPU and the GPU):
+// Method (own arithmetic: +, -, *, fma and the quotient and root below, which
+// all but always round as the CPU's / and sqrt do, so that with
+// -ffp-contract=off a CPU build with those gives the same bits):
 //   ENU -> ECEF: origin + R (e, n, u), R = the ENU basis in ECEF (the rotation
 //     pymap3d's enu2uvw applies);
 //   ECEF -> geodetic latitude and height: Bowring's iteration on the
@@ -37,16 +38,23 @@
 namespace vsm {
 namespace geo {
 
-// Division and square root for the magnitudes of this chain (1e-20 .. 1e20):
-// correctly rounded like / and sqrt, without the scaling that the general ones
-// do against over- and underflow, and with the reciprocal shared by quotients
-// of one divisor.  Two Newton steps on the hardware's estimate, then the
-// residual correction of Markstein (1990, IBM J. Res. Dev. 34:111); the root by
-// Goldschmidt's iteration with two residual corrections (ibid.).  A zero, an
-// infinity or a NaN where the chain divides makes NaN, and the point is
-// dropped as it is by / and sqrt.  The conversion is bound by its FP64
-// instructions, of which these take out a quarter (16.8 Mpx rasterised on the
-// UTM grid: 520 -> 413 us).
+// Division and square root for the magnitudes of this chain (1e-20 .. 1e20),
+// without the scaling that the general ones do against over- and underflow, and
+// with the reciprocal shared by quotients of one divisor.  Two Newton steps on
+// the hardware's estimate (off by at most 2^-24.3), then the residual
+// correction of Markstein (1990, IBM J. Res. Dev. 34:111); the root by
+// Goldschmidt's iteration with two residual corrections (ibid.).
+//
+// A quotient is at most half a unit in the last place and 2^-50 of one from
+// a / b, a root half and 2^-46 from sqrt(x): correctly rounded unless the value
+// lies that close to the middle between two numbers.  The reciprocal and the
+// inverse root would have to be correctly rounded for more.  The device's own /
+// and sqrt give the same bits there (4e6 pairs and 4e6 roots next to such a
+// middle: equal in all, 28024 quotients not correctly rounded by either) and
+// elsewhere (2.1e9 random pairs: equal in all).  A zero, an infinity or a NaN
+// where the chain divides makes NaN, and the point is dropped as it is by / and
+// sqrt.  The conversion is bound by its FP64 instructions, of which these take
+// out a quarter (16.8 Mpx rasterised on the UTM grid: 520 -> 413 us).
 VSM_GEO_FN double reciprocal(double b)
 {
     double y = __builtin_amdgcn_rcp(b);
