@@ -17,14 +17,15 @@ HIP = r"""
 #include <cstring>
 #include <mutex>
 #include <vector>
-enum hipError_t { hipSuccess = 0, hipErrorUnknown = 999 };
+enum hipError_t { hipSuccess = 0, hipErrorInvalidHandle = 400, hipErrorUnknown = 999 };
 enum hipMemcpyKind { hipMemcpyDeviceToHost = 2 };
 enum { hipEventDisableTiming = 2 };
 enum hipMemoryType { hipMemoryTypeUnregistered = 0, hipMemoryTypeHost = 1 };
 struct hipPointerAttribute_t { hipMemoryType type; };
 struct Op { void *dst; const void *src; size_t n; };
-struct Stream { std::mutex mu; std::vector<Op> ops; size_t done = 0; };
-struct Event { Stream *st = nullptr; size_t at = 0; bool bad = false; };
+struct Stream { std::mutex mu; std::vector<Op> ops; size_t done = 0; int device = 0; };
+struct Event { Stream *st = nullptr; size_t at = 0; bool bad = false; int device = 0; };
+inline thread_local int current = 0;               // the thread's device
 typedef Stream *hipStream_t;
 typedef Event *hipEvent_t;
 inline const char *marked = nullptr;               // reads of [marked, marked + marked_n) fail
@@ -51,6 +52,7 @@ inline hipError_t hipMemcpyAsync(void *d, const void *s, size_t n, hipMemcpyKind
 inline hipError_t hipEventRecord(hipEvent_t e, hipStream_t st)
 {
     std::lock_guard<std::mutex> lk(st->mu);
+    if (e->device != st->device) return hipErrorInvalidHandle;
     e->st = st; e->at = st->ops.size(); e->bad = is_marked(st->ops.back().src);
     return hipSuccess;
 }
@@ -65,7 +67,12 @@ inline hipError_t hipStreamSynchronize(hipStream_t st)
     std::lock_guard<std::mutex> lk(st->mu);
     return run_to(*st, st->ops.size());
 }
-inline hipError_t hipEventCreateWithFlags(hipEvent_t *e, unsigned) { *e = new Event; return hipSuccess; }
+inline hipError_t hipEventCreateWithFlags(hipEvent_t *e, unsigned) 
+{
+    *e = new Event;
+    (*e)->device = current;
+    return hipSuccess;
+}
 inline hipError_t hipEventDestroy(hipEvent_t e) { delete e; return hipSuccess; }
 inline hipError_t hipHostMalloc(void **p, size_t n, unsigned)
 {
@@ -80,7 +87,8 @@ inline hipError_t hipPointerGetAttributes(hipPointerAttribute_t *a, const void *
 }
 inline hipError_t hipHostFree(void *p) { free(p); return hipSuccess; }
 inline hipError_t hipGetLastError() { return hipSuccess; }
-inline hipError_t hipSetDevice(int) { return hipSuccess; }
+inline hipError_t hipSetDevice(int d) { current = d; return hipSuccess; }
+inline hipError_t hipGetDevice(int *d) { *d = current; return hipSuccess; }
 """
 
 MAIN = r"""
@@ -152,6 +160,24 @@ static int straight()
     return 0;
 }
 
+// The first copy of a context may come from a thread whose device is another
+// one (vsm_poll sets none), and leaves that as it is.
+static int other_device()
+{
+    CopyRing ring;
+    Stream st;
+    st.device = 3;
+    const size_t n = 3u << 20;
+    auto a = numbers(n, 5);
+    std::vector<unsigned char> d(n);
+    CopyCall call(ring, 3, &st);
+    CHECK(call.copy(d.data(), a.data(), n) == hipSuccess);
+    CHECK(call.finish() == hipSuccess);
+    CHECK(d == a);
+    CHECK(current == 0);
+    return 0;
+}
+
 // Calls of two threads, longer than the ring and in pieces of every kind.
 static int threads()
 {
@@ -175,7 +201,9 @@ static int threads()
 
 int main(int argc, char **argv)
 {
-    return argc > 1 && !strcmp(argv[1], "straight") ? straight() : errors() || early() || threads();
+    if (argc > 1 && !strcmp(argv[1], "straight")) return straight();
+    if (argc > 1 && !strcmp(argv[1], "device")) return other_device();
+    return errors() || early() || threads();
 }
 """
 
@@ -204,4 +232,11 @@ def test_copies_of_a_call_are_its_own(program):
 def test_pinned_memory_is_written_straight(program):
     """A destination that the device reaches itself does not go through the ring."""
     r = subprocess.run([program, "straight"], capture_output=True, text=True, timeout=60)
+    assert r.returncode == 0, r.stdout
+
+
+def test_ring_is_made_on_the_contexts_device(program):
+    """The ring's events belong to the device of the stream they are recorded
+    on, whichever device the calling thread uses."""
+    r = subprocess.run([program, "device"], capture_output=True, text=True, timeout=60)
     assert r.returncode == 0, r.stdout

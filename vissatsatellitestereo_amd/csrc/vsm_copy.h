@@ -144,12 +144,23 @@ private:
         return a.type != hipMemoryTypeUnregistered;
     }
 
-    // Makes the ring and the threads once; false where that failed.
+    // Makes the ring and the threads once; false where that failed.  The events
+    // have to belong to the device of the streams, which need not be the
+    // calling thread's.
     bool ready(int device)
     {
         std::lock_guard<std::mutex> lk(mu_);
         if (state_ != 0) return state_ > 0;
-        state_ = -1;
+        int before = device;
+        (void)hipGetDevice(&before);
+        (void)hipSetDevice(device);
+        state_ = make(device) ? 1 : -1;
+        (void)hipSetDevice(before);
+        return state_ > 0;
+    }
+
+    bool make(int device)
+    {
         void *p = nullptr;
         if (hipHostMalloc(&p, kSlots * kSlot, 0) != hipSuccess) {
             (void)hipGetLastError();
@@ -167,7 +178,6 @@ private:
             if (!threads_[0].joinable()) return false;
         }
         for (; n_free_ < kSlots; ++n_free_) free_[n_free_] = n_free_;
-        state_ = 1;
         return true;
     }
 
