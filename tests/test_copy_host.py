@@ -23,7 +23,7 @@ enum { hipEventDisableTiming = 2 };
 enum hipMemoryType { hipMemoryTypeUnregistered = 0, hipMemoryTypeHost = 1 };
 struct hipPointerAttribute_t { hipMemoryType type; };
 struct Op { void *dst; const void *src; size_t n; };
-struct Stream { std::mutex mu; std::vector<Op> ops; size_t done = 0; int device = 0; };
+struct Stream { std::mutex mu; std::vector<Op> ops; size_t done = 0; int device = 0; std::vector<size_t> waits; };
 struct Event { Stream *st = nullptr; size_t at = 0; bool bad = false; int device = 0; };
 inline thread_local int current = 0;               // the thread's device
 typedef Stream *hipStream_t;
@@ -31,9 +31,11 @@ typedef Event *hipEvent_t;
 inline const char *marked = nullptr;               // reads of [marked, marked + marked_n) fail
 inline size_t marked_n = 0;
 inline std::vector<std::pair<char *, size_t>> pinned;
+inline std::mutex pinned_mu;
 inline bool is_marked(const void *p) { return marked && (const char *)p >= marked && (const char *)p < marked + marked_n; }
 inline bool is_pinned(const void *p)
 {
+    std::lock_guard<std::mutex> lk(pinned_mu);
     for (auto &b : pinned) if ((const char *)p >= b.first && (const char *)p < b.first + b.second) return true;
     return false;
 }
@@ -65,6 +67,7 @@ inline hipError_t hipEventSynchronize(hipEvent_t e)
 inline hipError_t hipStreamSynchronize(hipStream_t st)
 {
     std::lock_guard<std::mutex> lk(st->mu);
+    st->waits.push_back(st->ops.size());
     return run_to(*st, st->ops.size());
 }
 inline hipError_t hipEventCreateWithFlags(hipEvent_t *e, unsigned) 
@@ -76,6 +79,7 @@ inline hipError_t hipEventCreateWithFlags(hipEvent_t *e, unsigned)
 inline hipError_t hipEventDestroy(hipEvent_t e) { delete e; return hipSuccess; }
 inline hipError_t hipHostMalloc(void **p, size_t n, unsigned)
 {
+    std::lock_guard<std::mutex> lk(pinned_mu);
     *p = malloc(n);
     pinned.emplace_back((char *)*p, n);
     return hipSuccess;
@@ -157,6 +161,7 @@ static int straight()
     CHECK(st.ops.size() == 1 && st.ops[0].dst == (char *)p + 64);
     CHECK(call.finish() == hipSuccess);
     CHECK(!memcmp((char *)p + 64, a.data(), n));
+    CHECK(hipHostFree(p) == hipSuccess);
     return 0;
 }
 
@@ -175,6 +180,26 @@ static int other_device()
     CHECK(call.finish() == hipSuccess);
     CHECK(d == a);
     CHECK(current == 0);
+    return 0;
+}
+
+// The caller waits for the work ahead, once a call, before the threads get any
+// of its copies to wait for.
+static int work_ahead()
+{
+    CopyRing ring;
+    Stream st;
+    const size_t n = 3u << 20;
+    auto a = numbers(n, 6);
+    std::vector<unsigned char> d(n), f(n);
+    char x = 1, y = 0;
+    CHECK(hipMemcpyAsync(&y, &x, 1, hipMemcpyDeviceToHost, &st) == hipSuccess);
+    CopyCall call(ring, 0, &st);
+    CHECK(call.copy(d.data(), a.data(), n) == hipSuccess);
+    CHECK(call.copy(f.data(), a.data(), n) == hipSuccess);
+    CHECK(st.waits.size() == 1 && st.waits[0] == 1);
+    CHECK(call.finish() == hipSuccess);
+    CHECK(d == a && f == a && y == 1);
     return 0;
 }
 
@@ -203,6 +228,7 @@ int main(int argc, char **argv)
 {
     if (argc > 1 && !strcmp(argv[1], "straight")) return straight();
     if (argc > 1 && !strcmp(argv[1], "device")) return other_device();
+    if (argc > 1 && !strcmp(argv[1], "ahead")) return work_ahead();
     return errors() || early() || threads();
 }
 """
@@ -239,4 +265,11 @@ def test_ring_is_made_on_the_contexts_device(program):
     """The ring's events belong to the device of the stream they are recorded
     on, whichever device the calling thread uses."""
     r = subprocess.run([program, "device"], capture_output=True, text=True, timeout=60)
+    assert r.returncode == 0, r.stdout
+
+
+def test_threads_do_not_wait_for_the_work_ahead(program):
+    """A thread that waits for an event keeps a core busy: the kernels ahead of
+    a copy are waited for by the caller alone."""
+    r = subprocess.run([program, "ahead"], capture_output=True, text=True, timeout=60)
     assert r.returncode == 0, r.stdout

@@ -48,6 +48,7 @@ private:
     int device_;
     hipStream_t st_;
     bool open_ = false;                        // copies queued and not waited for
+    bool waited_ = false;                      // the work ahead of the call's first ring copy is done
     int pending_ = 0;                          // of these, in the ring (guarded by its mutex, as error_)
     hipError_t error_ = hipSuccess;
 };
@@ -91,6 +92,14 @@ private:
     {
         if (n < kDirect || mapped(dst) || !ready(call.device_))
             return hipMemcpyAsync(dst, src, n, hipMemcpyDeviceToHost, call.st_);
+        // Waiting for an event takes a whole core, so the caller waits for the
+        // kernels ahead and the threads only for the DMA (DSM of 40 views, 44 ms:
+        // 163 ms of processor time a call where all of them waited).
+        if (!call.waited_) {
+            const hipError_t e = hipStreamSynchronize(call.st_);
+            if (e != hipSuccess) return e;
+            call.waited_ = true;
+        }
         // pieces of a short copy keep every thread busy; long ones take whole slots
         const size_t piece = std::min(kSlot, std::max(kPiece, (n / kThreadCount + kPage - 1) / kPage * kPage));
         for (size_t off = 0; off < n; off += piece) {
