@@ -254,6 +254,43 @@ def test_candidates_that_leave_change_nothing(tiny, ragged, many, name, n_src, e
     ctx.close()
 
 
+@pytest.mark.parametrize("name,n_src,extra", [
+    ("tiny", 3, dict(window_radius=3, window_step=1)),
+    ("many", 16, dict(window_radius=1, window_step=1, num_samples=4)),
+    ("many", 18, dict(window_radius=5, window_step=2, tile_width=16)),
+])
+def test_infinite_geometric_cost_changes_no_finite_one(tiny, many, name, n_src, extra):
+    """Steep normals: which variant a window pass takes depends on its planes,
+    so all of them are evaluated on every drawn source, also those whose cost
+    has become infinite (no depth in the source, no limit on the error).  A
+    limit too large for any plane to win with gives the same bits wherever the
+    winner's cost is finite."""
+    site = dict(tiny=tiny, many=many)[name]
+    p = _params(max_normal_angle=89.9, perturbation=3.0, **extra)
+    ctx, ref, srcs = _setup(site, p, 0, n_src)
+    rid, sids, dr = _id(site, ref), [_id(site, s) for s in srcs], site["dr"][ref]
+    for s, d in _src_depths(site, srcs).items():
+        ctx.set_depth_map(_id(site, s), d, kind=0)
+    st = ctx.debug_init(rid, sids, dr, 1)
+    H, W = site["imgs"][ref].shape
+    compared = 0
+    for k in range(6):
+        ctx.set_params(geom_consistency_max_cost=1e37)
+        o = ctx.debug_halfstep(rid, sids, dr, st, 1, k // 2, k % 2)
+        ctx.set_params(geom_consistency_max_cost=float("inf"))
+        g = ctx.debug_halfstep(rid, sids, dr, st, 1, k // 2, k % 2)
+        yy, xx = np.mgrid[0:H, 0:W]
+        ok = ((xx + yy) % 2 == k % 2).reshape(-1) & np.isfinite(g["cost"])
+        compared += int(ok.sum())
+        assert np.array_equal(g["cost"][ok], o["cost"][ok]), k
+        assert np.array_equal(g["depth"][ok], o["depth"][ok]), k
+        assert np.array_equal(g["normal"].reshape(-1, 3)[ok], o["normal"].reshape(-1, 3)[ok]), k
+        st = g
+    print("pixels compared", compared)
+    assert compared > H * W // 4
+    ctx.close()
+
+
 def test_lds_staged_costs_equal_cached(tiny):
     """The measurement kernel that reads window taps from LDS-staged boxes of
     the sources returns the same costs as its cached-gather twin and as

@@ -1192,7 +1192,7 @@ __device__ __forceinline__ void halfstep_tile(const ViewDesc &V, const Tile &t, 
             }
             uint32_t ids = part ? 0x765u : 0x4321u;
             int live = part ? kNHyp - 5 : kGroupH;
-            const float bound = prune ? best_s : INFINITY;
+            const float bound = best_s;
             for (int s = 0; s < S; ++s) {
                 const uint32_t e = s_list[s * kThreads + tid];
                 const int l = e ? live : 0;
@@ -1285,7 +1285,8 @@ __device__ __forceinline__ void halfstep_tile(const ViewDesc &V, const Tile &t, 
                     const float t = acc[k] + cnt * r;
                     acc[k] = k < l ? t : acc[k];
                 }
-                if (S > 1) drop_hyps(d, a, b, acc, ids, live, l, bound);
+                // not where nothing may leave: a sum may be infinite there
+                if (S > 1 && prune) drop_hyps(d, a, b, acc, ids, live, l, bound);
             }
 #pragma unroll
             for (int k = 0; k < kGroupH; ++k) {
