@@ -418,7 +418,7 @@ __global__ __launch_bounds__(256) void k_median3(const float *__restrict__ in, i
                                                  unsigned int first, float *__restrict__ out)
 {
     // one-dimensional grid from block `first` of the raster on: any number of rows
-    const unsigned int across = (e_size + 63) / 64, block = first + blockIdx.x;
+    const unsigned int across = ((unsigned int)e_size + 63u) / 64u, block = first + blockIdx.x;
     const int c = (int)(block % across) * 64 + (threadIdx.x & 63);
     const int r0 = ((int)(block / across) * 4 + (threadIdx.x >> 6)) * kMedRows;
     if (c >= e_size || r0 >= n_size) return;
@@ -727,9 +727,10 @@ hipError_t launch_view_dsm(const unsigned long long *keys, unsigned long long *c
 
 hipError_t launch_median3(const float *in, int e_size, int n_size, float *out, hipStream_t st)
 {
-    // A launch holds fewer than 2^32 threads.  Blocks are 64 columns wide, so a
-    // narrow raster of many rows has more threads than cells (2^28 rows of up to
-    // 8 cells reach the limit) and takes several launches.
+    // A launch holds fewer than 2^32 threads.  Blocks are 64 columns wide and 16
+    // rows high, so a raster that is narrower or lower has more threads than
+    // cells (2^28 rows of up to 8 cells and 2^30 columns of up to 2 reach the
+    // limit) and takes several launches.
     constexpr unsigned int kMaxBlocks = 1u << 23;
     const unsigned int blocks = nblk(e_size, 64) * nblk(n_size, 4 * kMedRows);
     for (unsigned int first = 0; first < blocks; first += kMaxBlocks) {
